@@ -440,43 +440,46 @@ int novaq_linear_backward(const float* grad, const float* x, int64_t N, int64_t 
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint8_t* base = static_cast<uint8_t*>(workspace);
   int rc = NOVAQ_OK;
-  // grad_weight = grad^T @ x: where the shape allows, the product that reads
-  // grad and x in place; it runs first, as it also leaves grad rounded to
-  // bf16 for grad_input's product (the rounding that product's staging would
-  // apply) and sums grad's columns into grad_bias
-  const bool tn = grad_weight && D_out > 0 && D_in > 0 && ws.tn;
-  uint16_t* g16 =
-      tn && grad_input && !ws.wn ? reinterpret_cast<uint16_t*>(base + ws.gyt) : nullptr;
+  if (N == 0 || D_in == 0 || D_out == 0) {  // empty sums
+    Epilogue ep{};
+    ep.out_dtype = F32;
+    if (grad_input && N > 0 && D_in > 0) {
+      rc = linear_launch(grad, F32, nullptr, N, 0, w_q, w_dtype, nullptr, ep, D_in, grad_input, s);
+      if (rc != NOVAQ_OK) return rc;
+    }
+    if (grad_weight && D_out > 0 && D_in > 0) {
+      rc = linear_launch(grad, F32, nullptr, D_out, 0, x, F32, nullptr, ep, D_in, grad_weight, s);
+      if (rc != NOVAQ_OK) return rc;
+    }
+    return grad_bias && D_out > 0 ? colsum_launch(grad, N, D_out, grad_bias, s) : rc;
+  }
+  // The products read the operands as they lie where that is the faster way:
+  // the 128 x 256-tile kernels (linear_tn_launch, linear_wn_launch) for shapes
+  // that fill the chip with such tiles, linear_split_kernel below that and for
+  // sides they do not take.  Otherwise: W's codes transposed and the forward
+  // product (E2M1 and 16-bit weights on wide tiles), and for fewer than 4
+  // features grad and x transposed as well.
+  const bool split = linear_split_bwd_supported(D_in, D_out);
+  const bool tn = grad_weight && linear_tn_preferred(D_out, D_in, N);
+  const bool wide = linear_wide_preferred(N, D_in);
+  const bool wn = grad_input && wide && linear_wn_takes(N, D_out, D_in, w_dtype);
+  const bool by_wt = grad_input && !wn &&
+                     (!split || (wide && w_dtype == E2M1 && D_out % 32 == 0) ||
+                      (wide && (w_dtype == BF16 || w_dtype == F16) && N % 128 == 0 &&
+                       D_in % 128 == 0 && D_out % 64 == 0));
+  // the tile product also leaves grad rounded to bf16 for grad_input's product
+  // (the rounding that product's staging would apply)
+  uint16_t* g16 = tn && by_wt ? reinterpret_cast<uint16_t*>(base + ws.gyt) : nullptr;
   bool bias_done = false;
   if (tn) {
     rc = linear_tn_launch(grad, x, D_out, D_in, N, grad_weight, grad_bias, g16, s);
-    if (rc != NOVAQ_OK) return rc;
     bias_done = true;
-  }
-  // grad_input = grad @ (s * dec(W)): where the shape allows, on W's FP8 codes
-  // read in place (transposing LDS reads) and the fp32 grad, rounded to bf16
-  // while staged; else the forward product on W^T (codes permuted) and the
-  // bf16 grad the weight-gradient product left
-  if (grad_input && N > 0 && D_in > 0) {
-    Epilogue ep{};
-    ep.out_dtype = F32;
-    if (ws.wn) {
-      rc = linear_wn_launch(grad, F32, N, D_out, w_q, w_dtype, w_scale, ep, D_in, grad_input, s);
-    } else {
-      void* wt = base + ws.wt;
-      rc = transpose_launch(w_q, w_dtype, D_out, D_in, wt, w_dtype, s);
-      if (rc != NOVAQ_OK) return rc;
-      if (g16)
-        rc = linear_launch(g16, BF16, nullptr, N, D_out, wt, w_dtype, w_scale, ep, D_in,
-                           grad_input, s);
-      else
-        rc = linear_launch(grad, N, D_out, wt, w_dtype, w_scale, nullptr, D_in, grad_input, s);
-    }
-    if (rc != NOVAQ_OK) return rc;
-  }
-  // otherwise the forward product of grad^T and x^T, both transposed straight
-  // to bf16 (the same round-to-nearest-even)
-  if (grad_weight && D_out > 0 && D_in > 0 && !tn) {
+  } else if (grad_weight && split) {
+    rc = linear_split_tn_launch(grad, x, D_out, D_in, N, grad_weight, grad_bias, s);
+    bias_done = true;
+  } else if (grad_weight) {
+    // the forward product of grad^T and x^T, both transposed straight to bf16
+    // (the same round-to-nearest-even)
     void* gyt = base + ws.gyt;
     void* xt = base + ws.xt;
     rc = transpose_launch(grad, F32, N, D_out, gyt, BF16, s);
@@ -486,10 +489,29 @@ int novaq_linear_backward(const float* grad, const float* x, int64_t N, int64_t 
     Epilogue ep{};
     ep.out_dtype = F32;
     rc = linear_launch(gyt, BF16, nullptr, D_out, N, xt, BF16, nullptr, ep, D_in, grad_weight, s);
+  }
+  if (rc != NOVAQ_OK) return rc;
+  if (grad_input) {
+    Epilogue ep{};
+    ep.out_dtype = F32;
+    if (wn) {
+      rc = linear_wn_launch(grad, F32, N, D_out, w_q, w_dtype, w_scale, ep, D_in, grad_input, s);
+    } else if (by_wt) {
+      void* wt = base + ws.wt;
+      rc = transpose_launch(w_q, w_dtype, D_out, D_in, wt, w_dtype, s);
+      if (rc != NOVAQ_OK) return rc;
+      if (g16)
+        rc = linear_launch(g16, BF16, nullptr, N, D_out, wt, w_dtype, w_scale, ep, D_in,
+                           grad_input, s);
+      else
+        rc = linear_launch(grad, N, D_out, wt, w_dtype, w_scale, nullptr, D_in, grad_input, s);
+    } else {
+      rc = linear_split_wcol_launch(grad, N, D_out, w_q, w_dtype, w_scale, D_in, grad_input, s);
+    }
     if (rc != NOVAQ_OK) return rc;
   }
   // grad_bias = grad summed over the batch
-  if (grad_bias && D_out > 0 && !bias_done) rc = colsum_launch(grad, N, D_out, grad_bias, s);
+  if (grad_bias && !bias_done) rc = colsum_launch(grad, N, D_out, grad_bias, s);
   return rc;
 }
 

@@ -25,6 +25,8 @@ extern template int linear_wn_launch_xt<BF16>(const uint8_t*, int64_t, int64_t, 
                                               const float*, const Epilogue&, int64_t, void*,
                                               hipStream_t);
 
+bool linear_wide_preferred(int64_t M, int64_t N) { return wide_preferred(M, N); }
+
 int linear_wn_launch(const void* x, int x_dtype, int64_t M, int64_t K, const void* w_q,
                      int w_dtype, const float* w_scale, const Epilogue& ep, int64_t N, void* y,
                      hipStream_t stream) {

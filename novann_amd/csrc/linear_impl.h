@@ -17,17 +17,26 @@
 //   - linear_f8_kernel (x stored as E4M3 / E5M2 and FP8 / FP4 weights, M % 128,
 //     N % 256, K % 128): both operands' codes on the FP8 MFMA
 //     (v_mfma_f32_32x32x64_f8f6f4), loaded straight into LDS;
-//   - linear_pingpong_kernel (FP8 weights, x in fp32 / bf16 / f16, M % 128,
-//     N % 256, K % 128): the 128 x 256 tile on two wave groups that take
-//     turns at the matrix cores and at the operand traffic;
-//   - linear_wide_kernel (E2M1 weights, and FP8 weights in their [K][N]
-//     layout for the backward; M % 128, N % 256, K % 128): one 128 x 256 tile
-//     per workgroup of 8 waves, K blocks of 128 (one 128-byte line of an FP8
-//     W row), W raw in LDS and decoded per MFMA fragment, buffer loads with
+//   - linear_pingpong_kernel (FP8 weights, x in fp32 / bf16 / f16, K % 16):
+//     the 128 x 256 tile on two wave groups that take turns at the matrix
+//     cores and at the operand traffic;
+//   - linear_wide_kernel (E2M1 weights, K % 32): one 128 x 256 tile per
+//     workgroup of 8 waves, K blocks of 128 (one 128-byte line of an FP8 W
+//     row), W raw in LDS and decoded per MFMA fragment, buffer loads with
 //     SGPR offsets;
-//   - linear_pipe_kernel (whole 128-row tiles, K % 64): W decoded once per
-//     workgroup into bf16 LDS tiles, loads kept up to 3 K blocks ahead;
-//   - linear_kernel: any shape (guarded edge tiles) and fp32 weights.
+//   - linear_pipe_kernel (16-bit weights, or FP8 x and W, in whole 128-row
+//     tiles, K % 64): W decoded once per workgroup into bf16 LDS tiles, loads
+//     kept up to 3 K blocks ahead;
+//   - linear_split_kernel (linear_split.h): any shape and format; small tiles
+//     with K split over the waves, for products of few rows or too few wide
+//     tiles to fill the chip, and for rows the others cannot read.
+// The ping-pong and wide kernels come in two forms: whole tiles, and RAG for
+// any M and N and a last K block that is not whole -- what lies past the
+// matrices is read as zeros through the buffer descriptors (the descriptors
+// cover whole rows; K past the end gets an offset outside them) and the
+// epilogue stores only what exists.  2000 x 4096 x 4096 (fp32 x, E4M3 W):
+// 448 us on the guarded-load kernel RAG replaced, 81.8 us now (2048 rows on
+// whole tiles: 67).
 // Tiles are numbered so that the workgroups the hardware sends to one XCD
 // (block id mod 8) cover a compact 4-row group of tiles, so their x rows and W
 // rows are shared through that XCD's L2.
@@ -36,6 +45,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "linear_split.h"
 #include "novaq_convert.h"
 #include "novaq_epilogue.h"
 #include "novaq_internal.h"
@@ -52,17 +62,13 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BM = 128, BN = 256, BK = 64;
-constexpr int LDS_ROW = BK + 8;  // bf16 per LDS row
-constexpr int THREADS = 256;
 constexpr int WM = 64, WN = 128;  // per-wave sub-tile
 constexpr int MT = WM / 32, NT = WN / 32;
-constexpr int XCH = BM * BK / 4 / THREADS;  // x 16-byte chunks per thread
 
 template <int WT>
 struct W {
   static constexpr int bits = dtype_bits(WT);
   static constexpr int epc = 128 / bits;           // elements per 16-byte chunk
-  static constexpr int chunks = BN * BK / epc / THREADS;  // per thread per K block
   static constexpr int words = epc / 2;            // bf16 pairs per chunk
 };
 
@@ -100,177 +106,6 @@ __device__ __forceinline__ void decode_chunk(const u32x4& c, uint32_t* out) {
       if (i % 2 == 0) out[i / 2] = f32x2_to_bf16(c[i], c[i + 1]);
     }
   }
-}
-
-// Element e of a row of W in storage order, for the guarded (edge) loads.
-template <int WT>
-__device__ __forceinline__ uint32_t load_w_elem(const uint8_t* row, int e) {
-  if constexpr (W<WT>::bits == 32) return reinterpret_cast<const uint32_t*>(row)[e];
-  else if constexpr (W<WT>::bits == 16) return reinterpret_cast<const uint16_t*>(row)[e];
-  else if constexpr (W<WT>::bits == 8) return row[e];
-  else return (row[e >> 1] >> ((e & 1) * 4)) & 0xFu;
-}
-
-// 16-byte chunk of row `r` (< rows) starting at element k (multiple of epc):
-// one vector load when it lies inside the row and rows are 16-byte aligned,
-// element loads with zero fill otherwise.
-template <int WT>
-__device__ __forceinline__ u32x4 load_w_chunk(const uint8_t* __restrict__ w, int r, int rows,
-                                              int k, int K, size_t row_bytes, bool vec_ok) {
-  constexpr int EPC = W<WT>::epc;
-  u32x4 v = {0u, 0u, 0u, 0u};
-  if (r >= rows) return v;
-  const uint8_t* row = w + (size_t)r * row_bytes;
-  if (vec_ok && k + EPC <= K) return *reinterpret_cast<const u32x4*>(row + (size_t)k * W<WT>::bits / 8);
-  constexpr int bits = W<WT>::bits;
-#pragma unroll
-  for (int e = 0; e < EPC; ++e) {
-    if (k + e < K) {
-      uint32_t c = load_w_elem<WT>(row, k + e);
-      v[(e * bits) / 32] |= c << ((e * bits) % 32);
-    }
-  }
-  return v;
-}
-
-// Raw codes of x elements k .. k+3 of row r (zeros past the row or matrix).
-template <int XT>
-__device__ __forceinline__ u32x4 load_x_chunk(const uint8_t* __restrict__ x, int r, int rows,
-                                              int k, int K, bool vec_ok) {
-  if (r >= rows) return u32x4{0u, 0u, 0u, 0u};
-  const int64_t e = (int64_t)r * K + k;
-  if (vec_ok && k + 4 <= K) return x4_raw<XT>(x, e);
-  return x4_raw_guarded<XT>(x, e, (int64_t)r * K + K);
-}
-
-template <int WT, int XT>
-__global__ __launch_bounds__(THREADS, 1) void linear_kernel(
-    const uint8_t* __restrict__ x, const float* __restrict__ x_scale, const uint8_t* __restrict__ w,
-    const float* __restrict__ w_scale,
-    Epilogue ep, void* __restrict__ y, int M, int N, int K, int tiles_m,
-    int tiles_n, int x_vec, int w_vec) {
-  __shared__ __attribute__((aligned(16))) __bf16 As[2][BM * LDS_ROW];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[2][BN * LDS_ROW];
-  using WTr = W<WT>;
-  constexpr int WCPR = BK / WTr::epc;  // W chunks per tile row
-  // rows of whole bytes: an odd-length E2M1 row ends with a pad nibble
-  const size_t w_row_bytes = ((size_t)K * WTr::bits + 7) / 8;
-
-  // tile index: XCD-contiguous, then 4-row groups walked column by column
-  const int T = tiles_m * tiles_n;
-  int t = blockIdx.x;
-  if ((T & 7) == 0) t = (t & 7) * (T >> 3) + (t >> 3);
-  constexpr int GM = 4;
-  const int group = t / (GM * tiles_n);
-  const int first_m = group * GM;
-  const int gm = min(tiles_m - first_m, GM);
-  const int rem = t - group * GM * tiles_n;
-  const int m0 = (first_m + rem % gm) * BM;
-  const int n0 = (rem / gm) * BN;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = (wave & 1) * WM, wn = (wave >> 1) * WN;
-
-  u32x4 xr[XCH];
-  u32x4 wr[WTr::chunks];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < XCH; ++i) {
-      int c = tid + THREADS * i;
-      xr[i] = load_x_chunk<XT>(x, m0 + (c >> 4), M, k0 + (c & 15) * 4, K, x_vec);
-    }
-#pragma unroll
-    for (int i = 0; i < WTr::chunks; ++i) {
-      int c = tid + THREADS * i;
-      wr[i] = load_w_chunk<WT>(w, n0 + c / WCPR, N, k0 + (c % WCPR) * WTr::epc, K, w_row_bytes,
-                               w_vec);
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < XCH; ++i) {
-      int c = tid + THREADS * i;
-      const xl_u32x2 pr = x4_bf16<XT>(xr[i]);
-      *reinterpret_cast<uint2*>(&As[buf][(c >> 4) * LDS_ROW + (c & 15) * 4]) = make_uint2(pr[0], pr[1]);
-    }
-#pragma unroll
-    for (int i = 0; i < WTr::chunks; ++i) {
-      int c = tid + THREADS * i;
-      uint32_t words[WTr::words];
-      decode_chunk<WT>(wr[i], words);
-      uint32_t* dst = reinterpret_cast<uint32_t*>(&Bs[buf][(c / WCPR) * LDS_ROW + (c % WCPR) * WTr::epc]);
-      if constexpr (WTr::words == 2) {
-        *reinterpret_cast<uint2*>(dst) = make_uint2(words[0], words[1]);
-      } else {
-#pragma unroll
-        for (int q = 0; q < WTr::words; q += 4)
-          *reinterpret_cast<uint4*>(dst + q) =
-              make_uint4(words[q], words[q + 1], words[q + 2], words[q + 3]);
-      }
-    }
-  };
-
-  f32x16 acc[MT][NT];
-#pragma unroll
-  for (int a = 0; a < MT; ++a)
-#pragma unroll
-    for (int b = 0; b < NT; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
-
-  const int kblocks = (K + BK - 1) / BK;
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  for (int kb = 0; kb < kblocks; ++kb) {
-    const int buf = kb & 1;
-    const bool more = kb + 1 < kblocks;
-    if (more) fetch((kb + 1) * BK);
-#pragma unroll
-    for (int s = 0; s < BK / 16; ++s) {
-      const int kk = s * 16 + (lane >> 5) * 8;
-      bf16x8 a[MT], b[NT];
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-        a[i] = *reinterpret_cast<const bf16x8*>(&As[buf][(wm + i * 32 + (lane & 31)) * LDS_ROW + kk]);
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-        b[j] = *reinterpret_cast<const bf16x8*>(&Bs[buf][(wn + j * 32 + (lane & 31)) * LDS_ROW + kk]);
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    if (more) stage(buf ^ 1);
-    __syncthreads();
-  }
-
-  // epilogue: lane holds column (lane & 31) and rows 8*(r/4) + 4*(lane/32) + r%4
-  const float s = product_scale(w_scale, x_scale);
-  const float inv_o = epi_inv_scale(ep);
-  uint32_t am = 0;
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int col = n0 + wn + j * 32 + (lane & 31);
-    if (col >= N) continue;
-    const EpiChan k = epi_chan(ep, col);
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < M) {
-          const float v = epi_value(ep, k, acc[i][j][r], s);
-          if (ep.amax) am = epi_track(am, v);
-          epi_store(ep.out_dtype, y, (size_t)row * N + col, v, inv_o);
-        }
-      }
-    }
-  }
-  epi_amax_commit(ep, am);
 }
 
 // Epilogue of a whole tile of 32 x 32 MFMA accumulators (acc[i][j]: rows
@@ -317,6 +152,51 @@ __device__ __forceinline__ void tile_epilogue(const Epilogue& ep, const f32x16 (
     case E4M3: am = store_tile<E4M3>(ep, acc, s, inv_o, z, y, N, row0, col0, lane); break;
     case E5M2: am = store_tile<E5M2>(ep, acc, s, inv_o, z, y, N, row0, col0, lane); break;
     default: am = store_tile<F32>(ep, acc, s, inv_o, z, y, N, row0, col0, lane); break;
+  }
+  epi_amax_commit(ep, am);
+}
+
+// tile_epilogue of a tile that may pass the matrix's last row or column (what
+// lies past them is not stored, nor tracked in the amax).
+template <int OD, int MTn, int NTn>
+__device__ __forceinline__ uint32_t store_tile_edge(const Epilogue& ep,
+                                                    const f32x16 (&acc)[MTn][NTn], float s,
+                                                    float inv_o, float z, void* y, int M, int N,
+                                                    int row0, int col0, int lane) {
+  uint32_t am = 0;
+  const int half = lane >> 5;
+#pragma unroll
+  for (int j = 0; j < NTn; ++j) {
+    const int col = col0 + j * 32 + (lane & 31);
+    if (col >= N) continue;
+    const EpiChan k = epi_chan(ep, col);
+#pragma unroll
+    for (int i = 0; i < MTn; ++i) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = row0 + i * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+        if (row >= M) continue;
+        const float v = epi_value_nb(k, acc[i][j][r], s, z);
+        am = epi_track(am, v);
+        epi_store_t<OD>(y, (size_t)row * N + col, v, inv_o);
+      }
+    }
+  }
+  return am;
+}
+
+template <int MTn, int NTn>
+__device__ __forceinline__ void tile_epilogue_edge(const Epilogue& ep,
+                                                   const f32x16 (&acc)[MTn][NTn], float s, void* y,
+                                                   int M, int N, int row0, int col0, int lane) {
+  const float inv_o = epi_inv_scale(ep), z = epi_relu_factor(ep);
+  uint32_t am;
+  switch (ep.out_dtype) {
+    case F16: am = store_tile_edge<F16>(ep, acc, s, inv_o, z, y, M, N, row0, col0, lane); break;
+    case BF16: am = store_tile_edge<BF16>(ep, acc, s, inv_o, z, y, M, N, row0, col0, lane); break;
+    case E4M3: am = store_tile_edge<E4M3>(ep, acc, s, inv_o, z, y, M, N, row0, col0, lane); break;
+    case E5M2: am = store_tile_edge<E5M2>(ep, acc, s, inv_o, z, y, M, N, row0, col0, lane); break;
+    default: am = store_tile_edge<F32>(ep, acc, s, inv_o, z, y, M, N, row0, col0, lane); break;
   }
   epi_amax_commit(ep, am);
 }
@@ -536,7 +416,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void linear_pipe_kernel(
 
 // ---------------------------------------------------------------------------
 // Wide-K kernel (dispatched for E2M1 weights; it also handles FP8, which the
-// ping-pong kernel below takes; K % 128 == 0): K blocks of 128, so one K
+// ping-pong kernel below takes): K blocks of 128, so one K
 // block of a W row is a whole 128-byte line for FP8 (64 bytes for E2M1) and
 // each W load fetches no line it uses only half of; barriers are
 // half as many.  W stays in its stored format in LDS (decoded per fragment),
@@ -554,7 +434,7 @@ struct Wide {
   static constexpr int cpr = row_bytes / 16;            // W 16-byte chunks per row
 };
 
-template <int WT, int XT>
+template <int WT, int XT, bool RAG>
 __global__ __launch_bounds__(512, 1) void linear_wide_kernel(
     const uint8_t* __restrict__ x, const float* __restrict__ x_scale, const uint8_t* __restrict__ w,
     const float* __restrict__ w_scale,
@@ -594,13 +474,15 @@ __global__ __launch_bounds__(512, 1) void linear_wide_kernel(
   // W: cpr chunks per row, NTH / cpr rows per pass.
   constexpr int XB = XL<XT>::bytes;
   const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(x + (size_t)m0 * K * XB), (short)0, BM * K * XB, 0x00020000);
+      const_cast<uint8_t*>(x + (size_t)m0 * K * XB), (short)0,
+      (RAG ? min(BM, M - m0) : BM) * K * XB, 0x00020000);
+  constexpr uint32_t OUT = 0x80000000u;  // a lane offset past any descriptor
   const uint32_t xlane = (uint32_t)((tid >> 5) * K + (tid & 31) * 4) * (uint32_t)XB;
   const uint32_t xstep = 16u * (uint32_t)K * (uint32_t)XB;
   const uint32_t w_row_bytes = (uint32_t)K * F::bits / 8;
   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(w + (size_t)n0 * w_row_bytes), (short)0, (int)(FBN * w_row_bytes),
-      0x00020000);
+      const_cast<uint8_t*>(w + (size_t)n0 * w_row_bytes), (short)0,
+      (int)((RAG ? min(FBN, N - n0) : FBN) * w_row_bytes), 0x00020000);
   const uint32_t wlane = (uint32_t)(tid / F::cpr) * w_row_bytes + (uint32_t)(tid % F::cpr) * 16u;
   const uint32_t wstep = (uint32_t)(NTH / F::cpr) * w_row_bytes;
 
@@ -625,22 +507,30 @@ __global__ __launch_bounds__(512, 1) void linear_wide_kernel(
     u32x4 w[WC];
   };
   auto fetch = [&](Regs& r, int kb) {
-    const uint32_t xk = (uint32_t)kb * (KB * XB);
-    const uint32_t wk = (uint32_t)kb * F::row_bytes;
+    // RAG: rows past the matrix and K past its end read zeros (the whole
+    // offset is the lane's, so the descriptor's range covers it)
+    uint32_t xo = xlane, wo = wlane, xk = (uint32_t)kb * (KB * XB), wk = (uint32_t)kb * F::row_bytes;
+    if constexpr (RAG) {
+      xo = kb * KB + (tid & 31) * 4 < K ? xlane + xk : OUT;
+      wo = (uint32_t)(kb * F::row_bytes + (tid % F::cpr) * 16) < w_row_bytes ? wlane + wk : OUT;
+      xk = wk = 0u;
+    }
 #pragma unroll
     for (int i = 0; i < XC; ++i) {
+      const uint32_t vo = RAG ? xo + i * xstep : xo, so = RAG ? 0u : xk + i * xstep;
       if constexpr (XB == 4) {
-        r.x[i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, xlane, xk + i * xstep, 0);
+        r.x[i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, vo, so, 0);
       } else if constexpr (XB == 2) {
-        const xl_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(xrs, xlane, xk + i * xstep, 0);
+        const xl_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(xrs, vo, so, 0);
         r.x[i] = u32x4{v[0], v[1], 0u, 0u};
       } else {
-        r.x[i] = u32x4{__builtin_amdgcn_raw_buffer_load_b32(xrs, xlane, xk + i * xstep, 0), 0u,
-                       0u, 0u};
+        r.x[i] = u32x4{__builtin_amdgcn_raw_buffer_load_b32(xrs, vo, so, 0), 0u, 0u, 0u};
       }
     }
 #pragma unroll
-    for (int i = 0; i < WC; ++i) r.w[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wlane, wk + i * wstep, 0);
+    for (int i = 0; i < WC; ++i)
+      r.w[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, RAG ? wo + i * wstep : wo,
+                                                     RAG ? 0u : wk + i * wstep, 0);
   };
   auto stage_units = [&](const Regs& r, const int BUF, int u0, int u1) {
 #pragma unroll
@@ -671,7 +561,7 @@ __global__ __launch_bounds__(512, 1) void linear_wide_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
 
-  const int kblocks = K / KB;
+  const int kblocks = RAG ? (K + KB - 1) / KB : K / KB;
   // Block kb in buffer BUF: fetch block kb+2 into `rf` (its block kb is in
   // LDS already), multiply, and stage block kb+1 from `rs` into buffer BUF^1
   // after MFMA steps 1..6.  Past the end the last block is fetched and staged
@@ -716,12 +606,13 @@ __global__ __launch_bounds__(512, 1) void linear_wide_kernel(
     if (kb + 1 < kblocks) body(kb + 1, 1, r1, r0);
   }
 
-  tile_epilogue(ep, acc, product_scale(w_scale, x_scale), y, N, m0 + wm, n0 + wn, lane);
+  const float s = product_scale(w_scale, x_scale);
+  if constexpr (RAG) tile_epilogue_edge(ep, acc, s, y, M, N, m0 + wm, n0 + wn, lane);
+  else tile_epilogue(ep, acc, s, y, N, m0 + wm, n0 + wn, lane);
 }
 
 // ---------------------------------------------------------------------------
-// Ping-pong kernel (E4M3 / E5M2 weights, x in fp32 / bf16 / f16, M % 128,
-// N % 256, K % 128): the wide kernel's 128 x 256 tile and 64 x 64 wave tiles,
+// Ping-pong kernel (E4M3 / E5M2 weights, x in fp32 / bf16 / f16): the wide kernel's 128 x 256 tile and 64 x 64 wave tiles,
 // scheduled so that the matrix cores are not idle while operands move.  The
 // 8 waves form two groups of 4 (rows 0-63 and 64-127 of the tile); waves w
 // and w + 4 share a SIMD.  Every wave runs the same program of phases
@@ -752,7 +643,7 @@ __global__ __launch_bounds__(512, 1) void linear_wide_kernel(
 // 32 lanes of a half-wave read 8 rows x 32 bytes, all in distinct banks) in
 // the MFMA's own K order, which the x fragments then follow.
 
-template <int WT, int XT, bool WN = false>
+template <int WT, int XT, bool WN = false, bool RAG = false>
 __global__ __launch_bounds__(512, 1) void linear_pingpong_kernel(
     const uint8_t* __restrict__ x, const float* __restrict__ x_scale, const uint8_t* __restrict__ w,
     const float* __restrict__ w_scale, Epilogue ep, void* __restrict__ y, int M, int N, int K,
@@ -797,8 +688,11 @@ __global__ __launch_bounds__(512, 1) void linear_pingpong_kernel(
 
   // x: the group's 64 rows, RP rows of 16-byte chunks per pass of its lanes
   const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(x + (size_t)(m0 + wm) * K * XB), (short)0, 64 * K * XB, 0x00020000);
+      const_cast<uint8_t*>(x + (size_t)(m0 + wm) * K * XB), (short)0,
+      (RAG ? max(0, min(64, M - m0 - wm)) : 64) * K * XB, 0x00020000);
+  constexpr uint32_t OUT = 0x80000000u;  // a lane offset past any descriptor
   const uint32_t xlane = (uint32_t)((gt / RL) * K + (gt % RL) * EPC) * (uint32_t)XB;
+  const int xk_lane = (gt % RL) * EPC;   // the lane's first K within a block
   const uint32_t xstep = (uint32_t)RP * (uint32_t)K * (uint32_t)XB;
   const int xw = (wm + gt / RL) * XP + (gt % RL) * EPC * 2;
 
@@ -811,11 +705,12 @@ __global__ __launch_bounds__(512, 1) void linear_pingpong_kernel(
       WN ? __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w + n0), (short)0,
                                              (int)((size_t)K * N - n0), 0x00020000)
          : __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w + (size_t)n0 * K), (short)0,
-                                             FBN * K, 0x00020000);
+                                             (RAG ? min(FBN, N - n0) : FBN) * K, 0x00020000);
   const uint32_t wlane =
       WN ? (uint32_t)((lane >> 4) * N + (((lane & 15) ^ (2 * (4 * (q & 1) + (lane >> 4)))) << 4))
          : (uint32_t)((lane >> 2) * K + (((lane & 3) ^ (lane >> 4)) << 4));
 
+  const int wcol = ((lane & 15) ^ (2 * (4 * (q & 1) + (lane >> 4)))) << 4;  // WN: its column
   // fragment bases: A row wm + la (+ 32 i), bytes 32 h (+ 64 t + 16 u) of
   // the row; B row wn + la (+ 32 j), chunk 2 t + h of the K half at slot
   // (2 t + h) ^ ((la / 4) % 4), so step t only flips address bit 5.  WN: A
@@ -828,7 +723,7 @@ __global__ __launch_bounds__(512, 1) void linear_pingpong_kernel(
       WN ? WOFF + (8 * h + bx) * 256 + (((4 * q + ((lane >> 4) & 1)) ^ (2 * bx)) << 4) + 8 * (lane & 1)
          : WOFF + (wn + la) * 64 + ((h ^ ((la >> 2) & 3)) << 4);
 
-  const int nb = K / KB;
+  const int nb = RAG ? (K + KB - 1) / KB : K / KB;
   u32x4 xr[2][XC];
   bf16x8 fa[2][2][MT];  // [32-K pair][step][M tile]
   u32x4 fb[2][FNT];     // [32-K pair][N tile]: 16 codes (WN: 8 per 16-K step)
@@ -842,9 +737,18 @@ __global__ __launch_bounds__(512, 1) void linear_pingpong_kernel(
 
   auto fetch_x = [&](u32x4 (&xs)[XC], int kb, const int i0, const int i1) {
     const uint32_t xk = (uint32_t)kb * (KB * XB);
+    if constexpr (RAG) {
+      // rows past M and K past the end read zeros (the whole offset is the
+      // lane's, so the descriptor's range covers it)
+      const uint32_t lo = kb * KB + xk_lane < K ? xlane + xk : OUT;
 #pragma unroll
-    for (int i = i0; i < i1; ++i)
-      xs[i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, xlane, xk + i * xstep, 0);
+      for (int i = i0; i < i1; ++i)
+        xs[i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, lo + i * xstep, 0, 0);
+    } else {
+#pragma unroll
+      for (int i = i0; i < i1; ++i)
+        xs[i] = __builtin_amdgcn_raw_buffer_load_b128(xrs, xlane, xk + i * xstep, 0);
+    }
   };
   auto stage_x = [&](const u32x4 (&xs)[XC], int slot, const int i0, const int i1) {
     uint8_t* d = lds + slot * XS + xw;
@@ -868,8 +772,18 @@ __global__ __launch_bounds__(512, 1) void linear_pingpong_kernel(
       const int j = 4 * i + q;
       const uint32_t so = WN ? (uint32_t)(kb * KB + 64 * hf + 4 * j) * (uint32_t)N
                              : (uint32_t)(16 * j) * (uint32_t)K + (uint32_t)kb * KB + 64u * hf;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_void*)(d + j * 64 * 16), 16, wlane, so,
-                                               0, 0);
+      if constexpr (RAG) {
+        // the lane's K row (WN) or 16-K chunk lies past K, or its column
+        // chunk (WN) or row past N: zeros
+        const int k = kb * KB + 64 * hf +
+                      (WN ? 4 * j + (lane >> 4) : (((lane & 3) ^ (lane >> 4)) << 4));
+        const bool in = k < K && (!WN || n0 + wcol < N);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_void*)(d + j * 64 * 16), 16,
+                                                 in ? wlane + so : OUT, 0, 0, 0);
+      } else {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_void*)(d + j * 64 * 16), 16, wlane, so,
+                                                 0, 0);
+      }
     }
   };
   auto read_frags = [&](int kb, const int hf) {
@@ -989,7 +903,9 @@ __global__ __launch_bounds__(512, 1) void linear_pingpong_kernel(
   if (g == 0) bar();  // both groups pass the same number of barriers
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  tile_epilogue(ep, acc, product_scale(w_scale, x_scale), y, N, m0 + wm, n0 + wn, lane);
+  const float s = product_scale(w_scale, x_scale);
+  if constexpr (RAG) tile_epilogue_edge(ep, acc, s, y, M, N, m0 + wm, n0 + wn, lane);
+  else tile_epilogue(ep, acc, s, y, N, m0 + wm, n0 + wn, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1230,80 +1146,102 @@ int launch_f8(const uint8_t* x, const float* x_scale, int64_t M, int64_t K, cons
   return check_launch();
 }
 
+// 128 x 256 tiles of an M x N product.
+inline int64_t wide_tiles(int64_t M, int64_t N) { return ((M + BM - 1) / BM) * ((N + 255) / 256); }
+
+// Whether 128 x 256 tiles are the better choice against linear_split_kernel's
+// small ones: where they cover more than an eighth of the CUs (K = 4096, fp32
+// x, E4M3 W: 256 x 4096 = 32 tiles 49.3 us here against 42.5 split, 512 x
+// 4096 = 64 tiles 49.8 against 81.6; 1024 x 1024 x 1024 = 32 tiles 17.0
+// against 15.1), and at most 64 rows (half a tile) always take the split.
+inline bool wide_preferred(int64_t M, int64_t N) {
+  return M > 64 && wide_tiles(M, N) > device_cu_count() / 8;
+}
+
 template <int WT, int XT>
 int launch(const uint8_t* x, const float* x_scale, int64_t M, int64_t K, const void* w,
            const float* w_scale, const Epilogue& ep, int64_t N, void* y, hipStream_t stream) {
-  const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  const int64_t T = tiles_m * tiles_n;
-  if (T > 0x7FFFFFFF || M > 0x7FFFFFFF || N > 0x7FFFFFFF || K > 0x7FFFFFFF) return NOVAQ_EINVAL;
+  const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + 255) / 256;
+  if (tiles_m * tiles_n > 0x7FFFFFFF || M > 0x7FFFFFFF || N > 0x7FFFFFFF || K > 0x7FFFFFFF)
+    return NOVAQ_EINVAL;
   const auto* wq = static_cast<const uint8_t*>(w);
   const bool rows_whole = M % BM == 0 && K > 0;
+  const bool whole = rows_whole && N % 256 == 0 && K % 128 == 0;
   if constexpr (dtype_bits(WT) <= 8 && (XT == E4M3 || XT == E5M2)) {
-    if (rows_whole && N % 256 == 0 && K % F8<WT, XT>::KS == 0)
-      return launch_f8<WT, XT>(x, x_scale, M, K, wq, w_scale, ep, N, y, stream);
+    if (whole) return launch_f8<WT, XT>(x, x_scale, M, K, wq, w_scale, ep, N, y, stream);
   }
-  if constexpr ((WT == E4M3 || WT == E5M2) && XL<XT>::bytes >= 2) {
-    // W tile (256 rows x K bytes) and x tile bytes must fit the buffer range
-    if (rows_whole && N % 256 == 0 && K % 128 == 0 && K <= (1 << 21)) {
-      hipLaunchKernelGGL((linear_pingpong_kernel<WT, XT>), dim3((unsigned)(tiles_m * (N / 256))),
-                         dim3(512), 0, stream, x, x_scale, wq, w_scale, ep, y, (int)M, (int)N,
-                         (int)K, (int)tiles_m, (int)(N / 256));
-      return check_launch();
+  const dim3 grid((unsigned)(tiles_m * tiles_n));
+  if (wide_preferred(M, N) && K > 0) {
+    // W tile (256 rows of K codes) and x tile bytes must fit the buffer range;
+    // ragged shapes need 16-byte chunks of W whole
+    if constexpr ((WT == E4M3 || WT == E5M2) && XL<XT>::bytes >= 2) {
+      if (K % 16 == 0 && K <= (1 << 21)) {
+        if (whole)
+          hipLaunchKernelGGL((linear_pingpong_kernel<WT, XT>), grid, dim3(512), 0, stream, x,
+                             x_scale, wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
+                             (int)tiles_n);
+        else
+          hipLaunchKernelGGL((linear_pingpong_kernel<WT, XT, false, true>), grid, dim3(512), 0,
+                             stream, x, x_scale, wq, w_scale, ep, y, (int)M, (int)N, (int)K,
+                             (int)tiles_m, (int)tiles_n);
+        return check_launch();
+      }
+    }
+    if constexpr (WT == E2M1) {
+      if (K % 32 == 0 && K <= (1 << 21)) {
+        if (whole)
+          hipLaunchKernelGGL((linear_wide_kernel<WT, XT, false>), grid, dim3(512), 0, stream, x,
+                             x_scale, wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
+                             (int)tiles_n);
+        else
+          hipLaunchKernelGGL((linear_wide_kernel<WT, XT, true>), grid, dim3(512), 0, stream, x,
+                             x_scale, wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
+                             (int)tiles_n);
+        return check_launch();
+      }
+    }
+    if constexpr (WT == BF16 || WT == F16 || (dtype_bits(WT) == 8 && XL<XT>::bytes == 1)) {
+      if (rows_whole && N % 256 == 0 && K % BK == 0) {
+        hipLaunchKernelGGL((linear_pipe_kernel<WT, XT, 256, 8, 1, 3>), grid, dim3(512), 0, stream,
+                           x, x_scale, wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
+                           (int)tiles_n);
+        return check_launch();
+      }
+      if (rows_whole && N % 128 == 0 && K % BK == 0) {
+        hipLaunchKernelGGL((linear_pipe_kernel<WT, XT, 128, 4, 2, 2>),
+                           dim3((unsigned)(tiles_m * (N / 128))), dim3(256), 0, stream, x, x_scale,
+                           wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
+                           (int)(N / 128));
+        return check_launch();
+      }
     }
   }
-  if constexpr (WT == E2M1) {
-    // tile byte sizes (BM * K * bytes(x) for x) must fit the 31-bit buffer range
-    if (rows_whole && N % 256 == 0 && K % 128 == 0 && K <= (1 << 21)) {
-      hipLaunchKernelGGL((linear_wide_kernel<WT, XT>), dim3((unsigned)(tiles_m * (N / 256))),
-                         dim3(512), 0, stream, x, x_scale, wq, w_scale, ep, y, (int)M, (int)N,
-                         (int)K, (int)tiles_m, (int)(N / 256));
-      return check_launch();
-    }
-  }
-  if constexpr (WT != F32) {
-    if (rows_whole && N % 256 == 0 && K % BK == 0) {
-      hipLaunchKernelGGL((linear_pipe_kernel<WT, XT, 256, 8, 1, 3>),
-                         dim3((unsigned)(tiles_m * (N / 256))), dim3(512), 0, stream, x, x_scale,
-                         wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m, (int)(N / 256));
-      return check_launch();
-    }
-    if (rows_whole && N % 128 == 0 && K % BK == 0) {
-      hipLaunchKernelGGL((linear_pipe_kernel<WT, XT, 128, 4, 2, 2>),
-                         dim3((unsigned)(tiles_m * (N / 128))), dim3(256), 0, stream, x, x_scale,
-                         wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m, (int)(N / 128));
-      return check_launch();
-    }
-  }
-  const int x_vec = (K % 4) == 0;
-  const int w_vec = ((K * W<WT>::bits / 8) % 16) == 0 && (K * W<WT>::bits) % 8 == 0;
-  hipLaunchKernelGGL((linear_kernel<WT, XT>), dim3((unsigned)T), dim3(THREADS), 0, stream, x,
-                     x_scale, wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
-                     (int)tiles_n, x_vec, w_vec);
-  return check_launch();
+  return split_launch<XT, false, WT, false>(x, x_scale, M, K, wq, w_scale, ep, N, y, nullptr, stream);
 }
 
 }  // namespace
 
 // y[M, N] = x[M, K] @ (s * dec(W[K, N])) with W in its natural [K][N] layout
 // (the Linear backward's grad_input = grad @ W on the forward's weight codes),
-// FP8 codes only, M % 128, N % 256, K % 128; NOVAQ_ENOTSUP for anything else
-// (the caller transposes W and uses the forward product instead).
+// FP8 codes only; NOVAQ_ENOTSUP for shapes linear_wn_takes refuses.
 template <int XT>
 int linear_wn_launch_xt(const uint8_t* x, int64_t M, int64_t K, const void* w_q, int w_dtype,
                         const float* w_scale, const Epilogue& ep, int64_t N, void* y,
                         hipStream_t stream) {
-  if (!linear_wn_supported(M, K, N, w_dtype)) return NOVAQ_ENOTSUP;
-  const int64_t tiles_m = M / BM, tiles_n = N / 256;
+  if (!linear_wn_takes(M, K, N, w_dtype)) return NOVAQ_ENOTSUP;
+  const int tm = (int)((M + BM - 1) / BM), tn = (int)((N + 255) / 256);
   const auto* wq = static_cast<const uint8_t*>(w_q);
+  const bool whole = linear_wn_supported(M, K, N, w_dtype);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)(tm * tn)), dim3(512), 0, stream, x, nullptr, wq,
+                       w_scale, ep, y, (int)M, (int)N, (int)K, tm, tn);
+    return check_launch();
+  };
   if (w_dtype == E4M3)
-    hipLaunchKernelGGL((linear_pingpong_kernel<E4M3, XT, true>),
-                       dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, stream, x, nullptr, wq,
-                       w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m, (int)tiles_n);
-  else
-    hipLaunchKernelGGL((linear_pingpong_kernel<E5M2, XT, true>),
-                       dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, stream, x, nullptr, wq,
-                       w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m, (int)tiles_n);
-  return check_launch();
+    return whole ? go(linear_pingpong_kernel<E4M3, XT, true, false>)
+                 : go(linear_pingpong_kernel<E4M3, XT, true, true>);
+  return whole ? go(linear_pingpong_kernel<E5M2, XT, true, false>)
+               : go(linear_pingpong_kernel<E5M2, XT, true, true>);
 }
 
 // The product for x stored as XT (one translation unit per XT instantiates it).

@@ -17,6 +17,10 @@
 // N % 256 and K % 32 are 0 and the tiles fill the GPU, else 128 x 256 (8 waves
 // of 64 x 64, K blocks of 64); two LDS stages.
 //
+// RAG takes any K and sides that are multiples of 4 (whole 4-element chunks):
+// what lies past the matrices is read as zeros through the buffer descriptor
+// and not stored.
+//
 // With a16 non-null the kernel also stores A rounded to bf16 (K x M, the
 // values it multiplies), each K block by one workgroup of the tile row (the
 // one whose column index is the block index mod the tiles per row), for a
@@ -76,7 +80,7 @@ __device__ __forceinline__ u32x4 load4(const __amdgpu_buffer_rsrc_t& rs, uint32_
   }
 }
 
-template <int AT, int BT, class C>
+template <int AT, int BT, class C, bool RAG>
 __global__ __launch_bounds__(C::NTH, 1) void linear_tn_kernel(const uint8_t* __restrict__ a,
                                                            const uint8_t* __restrict__ b,
                                                            float* __restrict__ c,
@@ -92,6 +96,8 @@ __global__ __launch_bounds__(C::NTH, 1) void linear_tn_kernel(const uint8_t* __r
   constexpr int RA = NTH / CA, RB = NTH / CB;  // rows per pass of the workgroup
   constexpr int AC = KB * CA / NTH, BC = KB * CB / NTH;  // chunks per thread
   constexpr int UNITS = AC + BC, STEPS = KB / 16;
+  // a lane offset past either operand: the load returns zeros
+  constexpr uint32_t OUT = 0x80000000u;
   static_assert(NTH % CA == 0 && NTH % CB == 0 && KB % RA == 0 && KB % RB == 0, "staging");
   __shared__ __attribute__((aligned(16))) uint8_t lds[2 * STAGE];
 
@@ -139,15 +145,28 @@ __global__ __launch_bounds__(C::NTH, 1) void linear_tn_kernel(const uint8_t* __r
     u32x4 a[AC];
     u32x4 b[BC];
   };
+  // RAG: chunks past M or N (whole chunks: both are multiples of 4) and rows
+  // past K carry an offset past the operand and read zeros
+  const bool a_in = !RAG || m0 + (tid % CA) * 4 < M, b_in = !RAG || n0 + (tid % CB) * 4 < N;
   auto fetch = [&](Regs& r, int kb) {
     const uint32_t ak = (uint32_t)kb * KB * (uint32_t)M * AB;
     const uint32_t bk = (uint32_t)kb * KB * (uint32_t)N * BB;
+    if constexpr (RAG) {
+      const int ra = K - kb * KB - tid / CA, rb = K - kb * KB - tid / CB;
 #pragma unroll
-    for (int i = 0; i < AC; ++i)
-      r.a[i] = load4<AB>(ars, alane, ak + i * astep);
+      for (int i = 0; i < AC; ++i)
+        r.a[i] = load4<AB>(ars, a_in && i * RA < ra ? alane + ak + i * astep : OUT, 0);
 #pragma unroll
-    for (int i = 0; i < BC; ++i)
-      r.b[i] = load4<BB>(brs, blane, bk + i * bstep);
+      for (int i = 0; i < BC; ++i)
+        r.b[i] = load4<BB>(brs, b_in && i * RB < rb ? blane + bk + i * bstep : OUT, 0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < AC; ++i)
+        r.a[i] = load4<AB>(ars, alane, ak + i * astep);
+#pragma unroll
+      for (int i = 0; i < BC; ++i)
+        r.b[i] = load4<BB>(brs, blane, bk + i * bstep);
+    }
   };
   const bool sums = colsum != nullptr && n0 == 0;
   float cs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -170,7 +189,8 @@ __global__ __launch_bounds__(C::NTH, 1) void linear_tn_kernel(const uint8_t* __r
         *reinterpret_cast<u32x2*>(lds + BUF * STAGE + aw + u * AW_STEP) = u32x2{p[0], p[1]};
         if (a16 && kbs >= 0 && kbs % tiles_n == ntile) {
           const int64_t row = (int64_t)kbs * KB + tid / CA + RA * u;
-          *reinterpret_cast<u32x2*>(a16 + row * M + m0 + (tid % CA) * 4) = u32x2{p[0], p[1]};
+          if (!RAG || (a_in && row < K))
+            *reinterpret_cast<u32x2*>(a16 + row * M + m0 + (tid % CA) * 4) = u32x2{p[0], p[1]};
         }
       } else {
         const int i = u - AC;
@@ -192,7 +212,7 @@ __global__ __launch_bounds__(C::NTH, 1) void linear_tn_kernel(const uint8_t* __r
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  const int kblocks = K / KB;
+  const int kblocks = RAG ? (K + KB - 1) / KB : K / KB;
   // Block kb in buffer BUF: fetch block kb+2 into `rf`, multiply, and stage
   // block kb+1 from `rs` into buffer BUF^1 over the steps; past the end the
   // last block is fetched and staged again into the idle buffer.
@@ -246,39 +266,67 @@ __global__ __launch_bounds__(C::NTH, 1) void linear_tn_kernel(const uint8_t* __r
       float v = part[col];
 #pragma unroll
       for (int t = 1; t < RA; ++t) v += part[t * BM + col];
-      colsum[m0 + col] = v;
+      if (!RAG || m0 + col < M) colsum[m0 + col] = v;
     }
   }
   Epilogue ep{};
   ep.out_dtype = F32;
-  tile_epilogue(ep, acc, 1.0f, c, N, m0 + wm, n0 + wn, lane);
+  if constexpr (RAG) tile_epilogue_edge(ep, acc, 1.0f, c, M, N, m0 + wm, n0 + wn, lane);
+  else tile_epilogue(ep, acc, 1.0f, c, N, m0 + wm, n0 + wn, lane);
 }
 
 }  // namespace
 
-bool linear_tn_supported(int64_t M, int64_t N, int64_t K) {
-  return M > 0 && N > 0 && K > 0 && M % Tn128::BM == 0 && N % Tn128::BN == 0 &&
-         K % Tn128::KB == 0 && K * M * 4 < ((int64_t)1 << 31) && K * N * 4 < ((int64_t)1 << 31);
+// Shapes the kernel takes at all, and whole tiles of it.
+static bool tn_takes(int64_t M, int64_t N, int64_t K) {
+  return M > 0 && N > 0 && K > 0 && M % 4 == 0 && N % 4 == 0 && K * M * 4 < ((int64_t)1 << 31) &&
+         K * N * 4 < ((int64_t)1 << 31);
 }
+static bool tn_whole(int64_t M, int64_t N, int64_t K) {
+  return M % Tn128::BM == 0 && N % Tn128::BN == 0 && K % Tn128::KB == 0;
+}
+
+bool linear_tn_supported(int64_t M, int64_t N, int64_t K) {
+  return tn_takes(M, N, K) && tn_whole(M, N, K);
+}
+
+// linear_split_kernel's small tiles win where 128 x 256 ones cover at most an
+// eighth of the CUs (K 512, fp32 grad and x: 1024 x 1024 = 32 tiles 14.4 us
+// here against 10.5, K 2048 45.5 against 24.7; 2048 x 2048 = 128 tiles 15.9
+// against 48).
+bool linear_tn_preferred(int64_t M, int64_t N, int64_t K) {
+  return tn_takes(M, N, K) &&
+         ((M + Tn128::BM - 1) / Tn128::BM) * ((N + Tn128::BN - 1) / Tn128::BN) >
+             device_cu_count() / 8;
+}
+
+namespace {
+
+template <class C, bool RAG>
+int tn_launch_tile(const float* a, const float* b, int64_t M, int64_t N, int64_t K, float* c,
+                   float* colsum, uint16_t* a16, hipStream_t stream) {
+  const int tm = (int)((M + C::BM - 1) / C::BM), tn = (int)((N + C::BN - 1) / C::BN);
+  hipLaunchKernelGGL((linear_tn_kernel<F32, F32, C, RAG>), dim3((unsigned)(tm * tn)), dim3(C::NTH),
+                     0, stream, reinterpret_cast<const uint8_t*>(a),
+                     reinterpret_cast<const uint8_t*>(b), c, colsum, a16, (int)M, (int)N, (int)K, tm,
+                     tn);
+  return check_launch();
+}
+
+}  // namespace
 
 int linear_tn_launch(const float* a, const float* b, int64_t M, int64_t N, int64_t K, float* c,
                      float* colsum, uint16_t* a16, hipStream_t stream) {
-  if (!linear_tn_supported(M, N, K)) return NOVAQ_ESHAPE;
-  const uint8_t* ap = reinterpret_cast<const uint8_t*>(a);
-  const uint8_t* bp = reinterpret_cast<const uint8_t*>(b);
-  if (M % Tn256::BM == 0 && N % Tn256::BN == 0 && K % Tn256::KB == 0 &&
-      (M / Tn256::BM) * (N / Tn256::BN) >= device_cu_count()) {
-    const int tm = (int)(M / Tn256::BM), tn = (int)(N / Tn256::BN);
-    hipLaunchKernelGGL((linear_tn_kernel<F32, F32, Tn256>), dim3((unsigned)(tm * tn)),
-                       dim3(Tn256::NTH), 0, stream, ap, bp, c, colsum, a16, (int)M, (int)N, (int)K, tm,
-                       tn);
-  } else {
-    const int tm = (int)(M / Tn128::BM), tn = (int)(N / Tn128::BN);
-    hipLaunchKernelGGL((linear_tn_kernel<F32, F32, Tn128>), dim3((unsigned)(tm * tn)),
-                       dim3(Tn128::NTH), 0, stream, ap, bp, c, colsum, a16, (int)M, (int)N, (int)K, tm,
-                       tn);
+  if (!tn_takes(M, N, K)) return NOVAQ_ESHAPE;
+  const int64_t tiles256 = ((M + Tn256::BM - 1) / Tn256::BM) * ((N + Tn256::BN - 1) / Tn256::BN);
+  if (tn_whole(M, N, K)) {
+    if (M % Tn256::BM == 0 && tiles256 >= device_cu_count())
+      return tn_launch_tile<Tn256, false>(a, b, M, N, K, c, colsum, a16, stream);
+    return tn_launch_tile<Tn128, false>(a, b, M, N, K, c, colsum, a16, stream);
   }
-  return check_launch();
+  if (tiles256 >= device_cu_count())
+    return tn_launch_tile<Tn256, true>(a, b, M, N, K, c, colsum, a16, stream);
+  return tn_launch_tile<Tn128, true>(a, b, M, N, K, c, colsum, a16, stream);
 }
 
 }  // namespace novaq

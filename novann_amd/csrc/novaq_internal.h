@@ -80,12 +80,16 @@ int linear_launch(const void* x, int x_dtype, const float* x_scale, int64_t N, i
                   const void* w_q, int w_dtype, const float* w_scale, const Epilogue& ep,
                   int64_t D_out, void* y, hipStream_t stream);
 // y[M, N] = x[M, K] @ (s * dec(W[K, N])) with W's codes in their natural
-// [K][N] layout (no transposed copy): bf16 x, FP8 W, M % 128, N % 256,
-// K % 128; NOVAQ_ENOTSUP otherwise.
+// [K][N] layout (no transposed copy): fp32 or bf16 x, FP8 W, N a multiple of
+// 16 and K of 8 (linear_wn_takes); linear_wn_supported: the shapes made of
+// whole tiles (M % 128, N % 256, K % 128).  NOVAQ_ENOTSUP otherwise.
+inline bool linear_wn_takes(int64_t M, int64_t K, int64_t N, int w_dtype) {
+  return (w_dtype == 3 || w_dtype == 4) && M > 0 && M <= 0x7FFFFFFF && N > 0 && N % 16 == 0 &&
+         K > 0 && K % 8 == 0 && K <= (1 << 21) && K * N < ((int64_t)1 << 31) &&
+         ((M + 127) / 128) * ((N + 255) / 256) <= 0x7FFFFFFF;
+}
 inline bool linear_wn_supported(int64_t M, int64_t K, int64_t N, int w_dtype) {
-  return (w_dtype == 3 || w_dtype == 4) && M > 0 && M % 128 == 0 && M <= 0x7FFFFFFF &&
-         N > 0 && N % 256 == 0 && K > 0 && K % 128 == 0 && K <= (1 << 21) &&
-         K * N < ((int64_t)1 << 31);
+  return linear_wn_takes(M, K, N, w_dtype) && M % 128 == 0 && N % 256 == 0 && K % 128 == 0;
 }
 int linear_wn_launch(const void* x, int x_dtype, int64_t M, int64_t K, const void* w_q,
                      int w_dtype, const float* w_scale, const Epilogue& ep, int64_t N, void* y,
@@ -142,12 +146,28 @@ int transpose_launch(const void* src, int st, int64_t rows, int64_t cols, void* 
 
 // c[M, N] = sum over k of a[k, m] * b[k, n] (a: K x M, b: K x N, row-major
 // fp32), both rounded to bf16, fp32 sums: the Linear weight gradient without
-// transposed copies.  Shapes: M % 128, N % 256, K % 64, K * M and K * N
-// fp32 bytes under 2 GiB.  colsum (optional): colsum[m] = sum over k of
+// transposed copies.  Shapes: M and N multiples of 4, K * M and K * N fp32
+// bytes under 2 GiB.  linear_tn_supported: those made of whole tiles (M % 128,
+// N % 256, K % 64); linear_tn_preferred: those it is the faster kernel for
+// (against linear_split_tn_launch).  colsum (optional): colsum[m] = sum over k of
 // a[k, m] in fp32, in a fixed order.  a16 (optional): a rounded to bf16.
 bool linear_tn_supported(int64_t M, int64_t N, int64_t K);
+bool linear_tn_preferred(int64_t M, int64_t N, int64_t K);
 int linear_tn_launch(const float* a, const float* b, int64_t M, int64_t N, int64_t K, float* c,
                      float* colsum, uint16_t* a16, hipStream_t stream);
+
+// The backward's products on operands as they lie, any M, any K (D_in and
+// D_out at least 4, even for E2M1): y[M, N] = grad[M, K] @ (s * dec(W[K, N])),
+// and c[M, N] = sum over k of a[k, m] * b[k, n] with the optional fp32 colsum
+// as linear_tn_launch gives it (another fixed order).
+// linear_wide_preferred: the 128 x 256-tile kernels are the faster ones for an
+// M x N product of a shape they take.
+bool linear_wide_preferred(int64_t M, int64_t N);
+bool linear_split_bwd_supported(int64_t D_in, int64_t D_out);
+int linear_split_wcol_launch(const float* grad, int64_t M, int64_t K, const void* w_q, int w_dtype,
+                             const float* w_scale, int64_t N, float* y, hipStream_t stream);
+int linear_split_tn_launch(const float* a, const float* b, int64_t M, int64_t N, int64_t K,
+                           float* c, float* colsum, hipStream_t stream);
 
 // Workspace parts of conv2d_backward_launch (byte offsets, 256-byte aligned):
 // the flipped weights, the grad_weight partials (chunks x C_out x C*KH*KW
