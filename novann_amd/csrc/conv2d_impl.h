@@ -37,6 +37,7 @@
 
 #include <algorithm>
 
+#include "conv2d_gather.h"
 #include "novaq_convert.h"
 #include "novaq_epilogue.h"
 #include "novaq_internal.h"
@@ -1632,6 +1633,28 @@ bool launch_smallc(const uint8_t* x, const float* x_scale, const void* w, const 
   return true;
 }
 
+// The gathered path where it takes the shape; returns false otherwise.
+template <int WT, int XT>
+bool launch_gather(const uint8_t* x, const float* x_scale, const void* w, const float* w_scale,
+                   const Epilogue& ep, void* y, const ConvGeom& cg, hipStream_t stream, int* rc) {
+  if (cg.pad_mode != NOVAQ_PAD_ZEROS && (cg.ph || cg.pw)) return false;
+  if (!gather_takes<WT, XT>(cg.C_out, cg.C, cg.H, cg.W, (int64_t)cg.KH * cg.KW, cg.N,
+                            (int64_t)cg.OH * cg.OW))
+    return false;
+  GatherGeom g{};
+  g.M = cg.C_out;
+  g.K = cg.C * cg.KH * cg.KW;
+  g.KH = cg.KH; g.KW = cg.KW;
+  g.GH = cg.H; g.GW = cg.W;
+  g.PH = cg.OH; g.PW = cg.OW;
+  g.sh = cg.sh; g.sw = cg.sw; g.ph = cg.ph; g.pw = cg.pw;
+  g.gathered = cg.C * cg.H * cg.W;
+  g.images = cg.N;
+  *rc = gather_launch<WT, XT>(x, x_scale, static_cast<const uint8_t*>(w), w_scale, ep, y, g,
+                                     stream);
+  return true;
+}
+
 template <int WT, int XT>
 int launch(const uint8_t* x, const float* x_scale, const void* w, const float* w_scale,
            const Epilogue& ep, void* y, ConvGeom g, hipStream_t stream) {
@@ -1649,21 +1672,31 @@ int launch(const uint8_t* x, const float* x_scale, const void* w, const float* w
       return check_launch();
     }
   }
-  {
-    BandGeom b;
-    size_t lds = 0;
-    int ipt = 0;
-    if (band_geometry<WT>(g, b, lds, &ipt, ep.out_dtype)) {
-      const int64_t co_blocks = (g.C_out + CO_TILE - 1) / CO_TILE;
-      if constexpr (group_bytes<WT>() < 16) {
-        if (b.taps == 9 && g.C % 8 == 0 && b.raw_ok) {
-          if (ipt == 1) return launch_band<WT, XT, 1, true>(x, x_scale, w, w_scale, ep, y, b, lds, co_blocks, stream);
-          return launch_band<WT, XT, 0, true>(x, x_scale, w, w_scale, ep, y, b, lds, co_blocks, stream);
-        }
+  BandGeom b;
+  size_t band_lds = 0;
+  int ipt = 0;
+  const bool band = band_geometry<WT>(g, b, band_lds, &ipt, ep.out_dtype);
+  const int64_t co_blocks = (g.C_out + CO_TILE - 1) / CO_TILE;
+  // The gathered path wherever no band fits in LDS, and where bands would
+  // leave CUs idle (64 -> 64 channels, 3 x 3, 16 maps of 14 x 14 = 16 bands:
+  // 11.2 us gathered, 23.1 in bands; 400 bands of 16 -> 48 channels 28.6
+  // against 17.7) or fill a CU with fewer than four workgroups of a large
+  // window's weights (32 -> 64, 5 x 5, 64 maps of 28 x 28: 31.2 against 49.3).
+  if (!band || (int64_t)g.N * b.bands * co_blocks < device_cu_count() ||
+      (band_lds > BAND_LDS_FOUR && b.taps > 9)) {
+    int rc = NOVAQ_OK;
+    if (launch_gather<WT, XT>(x, x_scale, w, w_scale, ep, y, g, stream, &rc)) return rc;
+  }
+  if (band) {
+    const size_t lds = band_lds;
+    if constexpr (group_bytes<WT>() < 16) {
+      if (b.taps == 9 && g.C % 8 == 0 && b.raw_ok) {
+        if (ipt == 1) return launch_band<WT, XT, 1, true>(x, x_scale, w, w_scale, ep, y, b, lds, co_blocks, stream);
+        return launch_band<WT, XT, 0, true>(x, x_scale, w, w_scale, ep, y, b, lds, co_blocks, stream);
       }
-      if (ipt == 1) return launch_band<WT, XT, 1, false>(x, x_scale, w, w_scale, ep, y, b, lds, co_blocks, stream);
-      return launch_band<WT, XT, 0, false>(x, x_scale, w, w_scale, ep, y, b, lds, co_blocks, stream);
     }
+    if (ipt == 1) return launch_band<WT, XT, 1, false>(x, x_scale, w, w_scale, ep, y, b, lds, co_blocks, stream);
+    return launch_band<WT, XT, 0, false>(x, x_scale, w, w_scale, ep, y, b, lds, co_blocks, stream);
   }
   // staged rows for a run of PIX_TILE pixels: it spans at most
   // ceil((PIX_TILE - 1) / OW) + 1 output rows
@@ -1702,7 +1735,6 @@ int launch(const uint8_t* x, const float* x_scale, const void* w, const float* w
     if (e != hipSuccess) return hip_fail(e);
     lds_enabled = LDS_LIMIT;
   }
-  const int64_t co_blocks = (g.C_out + CO_TILE - 1) / CO_TILE;
   int64_t grid = (int64_t)device_cu_count() * CONV_OCC;
   if (grid > g.tiles) grid = g.tiles;
   if (grid < 1) grid = 1;

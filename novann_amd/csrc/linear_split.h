@@ -124,8 +124,9 @@ struct LsRow {
   static constexpr bool HALF = bits >= 16;
   static constexpr int NE = HALF ? 8 : 16;        // elements a load takes
   static constexpr int NW = NE * bits / 32;       // words of them
+  typedef uint32_t Run __attribute__((ext_vector_type(NW)));
   struct Regs {
-    uint32_t w[T][NW];
+    Run w[T];
   };
   const uint8_t* row[T];
   int kl;  // the lane's first element within a block
@@ -141,17 +142,13 @@ struct LsRow {
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       const uint8_t* p = row[t] + b;
-      if constexpr (NW == 2) {
-        const ls_u32x2u v = *reinterpret_cast<const ls_u32x2u*>(p);
-        r.w[t][0] = v[0];
-        r.w[t][1] = v[1];
+      if constexpr (NW == 8) {
+        const ls_u32x4u lo = *reinterpret_cast<const ls_u32x4u*>(p);
+        const ls_u32x4u hi = *reinterpret_cast<const ls_u32x4u*>(p + 16);
+        r.w[t] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       } else {
-#pragma unroll
-        for (int q = 0; q < NW / 4; ++q) {
-          const ls_u32x4u v = *reinterpret_cast<const ls_u32x4u*>(p + 16 * q);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) r.w[t][4 * q + e] = v[e];
-        }
+        typedef Run RunU __attribute__((aligned(1)));
+        r.w[t] = *reinterpret_cast<const RunU*>(p);
       }
     }
   }
@@ -170,9 +167,40 @@ struct LsRow {
       }
     }
   }
+  // load_tail for K >= NE (even for 4-bit codes) with few instructions: a run
+  // that would pass K is read ending at K and shifted down to its place, zeros
+  // behind it.
+  __device__ __forceinline__ void load_end(Regs& r, int k0, const int u, int K) const {
+    const int k = k0 + kl + 8 * u;
+    const int from = min(k, K - NE), d = min(k - from, NE);  // elements to drop
+    const int64_t b = (int64_t)from * bits / 8;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      uint32_t w[NW];
+      const uint8_t* p = row[t] + b;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) w[i] = *reinterpret_cast<const ls_u32u*>(p + 4 * i);
+      const int sh = d * bits, words = sh >> 5, rest = sh & 31;
+#pragma unroll
+      for (int step = 1; step < 2 * NW; step *= 2) {
+#pragma unroll
+        for (int i = 0; i < NW; ++i)
+          w[i] = (words & step) ? (i + step < NW ? w[i + step] : 0u) : w[i];
+      }
+#pragma unroll
+      for (int i = 0; i < NW; ++i)
+        w[i] = rest ? (w[i] >> rest) | (i + 1 < NW ? w[i + 1] << (32 - rest) : 0u) : w[i];
+#pragma unroll
+      for (int i = 0; i < NW; ++i) r.w[t][i] = w[i];
+    }
+  }
   // tile t's fragment of step u
   static __device__ __forceinline__ ls_bf16x8 frag(const Regs& r, const int t, const int u) {
-    return ls_decode8<DT>(&r.w[t][HALF ? 0 : u * NW / 2]);
+    constexpr int N8 = bits / 4;  // words of 8 elements
+    uint32_t w[N8];
+#pragma unroll
+    for (int i = 0; i < N8; ++i) w[i] = r.w[t][(HALF ? 0 : u * N8) + i];
+    return ls_decode8<DT>(w);
   }
   // index of the operand's element that tile t, lane row r holds
   __device__ __forceinline__ int index(const int t, int r) const { return 16 * t + r; }
