@@ -490,6 +490,52 @@ __global__ __launch_bounds__(256) void global_avg_pool2d_plane_kernel(
   if (lane == 0) y[plane] = total / (float)hw;
 }
 
+// K x K windows (K = 2, 3) with zeros padding: lane t makes output element t
+// from K * K buffer loads issued together; a tap on the padding carries an
+// offset past the descriptor and reads 0, the padding's +0 code.  t < 2^31.
+// Measured (256 x 64 planes of 28 x 28, fp32): 3 x 3 / 2 with padding 18.1 us,
+// 32.6 on max_pool2d_kernel's run-time window; 3 x 3 / 1 45.9 us (108).
+template <int XT, int K>
+__global__ __launch_bounds__(256) void max_pool2d_win_kernel(const uint8_t* __restrict__ x,
+                                                            uint8_t* __restrict__ y, PoolGeom g,
+                                                            FastDiv dwin, FastDiv dow,
+                                                            uint32_t total) {
+  constexpr int EB = XL<XT>::bits / 8;
+  constexpr uint32_t OUT = 0x80000000u;
+  const uint32_t npix = (uint32_t)(g.OH * g.OW);
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+  // offsets are relative to the workgroup's first plane
+  const uint32_t plane0 = fdiv(blockIdx.x * 256u, dwin);
+  const int64_t hw = (int64_t)g.H * g.W;
+  const int64_t left = (g.N * g.C - plane0) * hw * EB;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(x + (int64_t)plane0 * hw * EB), (short)0,
+      (int)(left < 0x7FFFFFFF ? left : 0x7FFFFFFF), 0x00020000);
+  const uint32_t plane = fdiv(t, dwin), pix = t - plane * npix;
+  const int oh = (int)fdiv(pix, dow), ow = (int)pix - oh * g.OW;
+  const int h0 = oh * g.sh - g.ph, w0 = ow * g.sw - g.pw;
+  const uint32_t base = (plane - plane0) * (uint32_t)hw + (uint32_t)(h0 * g.W + w0);
+  uint32_t c[K * K];
+#pragma unroll
+  for (int a = 0; a < K; ++a) {
+    const bool row = (unsigned)(h0 + a) < (unsigned)g.H;
+#pragma unroll
+    for (int b = 0; b < K; ++b) {
+      const bool in = row && (unsigned)(w0 + b) < (unsigned)g.W;
+      const uint32_t at = in && t < total ? (base + (uint32_t)(a * g.W + b)) * EB : OUT;
+      if constexpr (EB == 4) c[a * K + b] = __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0);
+      else if constexpr (EB == 2) c[a * K + b] = __builtin_amdgcn_raw_buffer_load_b16(rs, at, 0, 0);
+      else c[a * K + b] = __builtin_amdgcn_raw_buffer_load_b8(rs, at, 0, 0);
+    }
+  }
+  if (t >= total) return;
+  uint32_t best = c[0];
+  float bv = u2f(decode<XT>(best));
+#pragma unroll
+  for (int k = 1; k < K * K; ++k) take_max(c[k], u2f(decode<XT>(c[k])), best, bv);
+  store_code<XT>(y, t, best);
+}
+
 template <int XT>
 int launch_max(const void* x, void* y, const PoolGeom& g, hipStream_t stream) {
   const int64_t npix = (int64_t)g.OH * g.OW;
@@ -529,6 +575,17 @@ int launch_max(const void* x, void* y, const PoolGeom& g, hipStream_t stream) {
                          (uint32_t)items);
       return check_launch();
     }
+  }
+  const int64_t outs = g.N * g.C * npix;
+  if (g.KH == g.KW && (g.KH == 2 || g.KH == 3) &&
+      (g.pad_mode == NOVAQ_PAD_ZEROS || (g.ph == 0 && g.pw == 0)) &&
+      outs < ((int64_t)1 << 31) - 256 &&
+      (256 / npix + 2) * (int64_t)g.H * g.W * (int64_t)EB < 0x7FFFFFFF) {
+    auto kern = g.KH == 2 ? max_pool2d_win_kernel<XT, 2> : max_pool2d_win_kernel<XT, 3>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, stream,
+                       static_cast<const uint8_t*>(x), static_cast<uint8_t*>(y), g,
+                       fast_div((uint32_t)npix), fast_div((uint32_t)g.OW), (uint32_t)outs);
+    return check_launch();
   }
   const int64_t blocks = (g.N * g.C * npix + 255) / 256;
   if (blocks > 0x7FFFFFFF) return NOVAQ_EINVAL;
@@ -682,6 +739,228 @@ __global__ __launch_bounds__(256) void max_pool2d_bwd_kernel(const float* __rest
   gi[t] = sum;
 }
 
+// The max pool's backward on planes that fit in LDS: a workgroup takes P whole
+// planes (about 2048 elements) and stages them padded in fp32 -- the padding
+// mode resolved once an element instead of once a window tap -- with 4-element
+// loads; x and grad are then read from memory once.
+struct PoolTile {
+  PoolGeom g;
+  int64_t planes;
+  int P;             // planes of a workgroup
+  int hp, wp;        // padded plane
+  int vec;           // 4-element loads (and 16-byte gradient stores)
+  int rows4;         // W % 4 == 0: a 4-element group lies in one row
+  FastDiv fd_hw, fd_w, fd_pad, fd_wp, fd_win, fd_ow, fd_sh, fd_sw;
+};
+
+// A workgroup's bytes of LDS per plane: the values, and (maximum, quotient) of
+// each window.
+inline int64_t pool_tile_bytes(const PoolGeom& g) {
+  return ((int64_t)g.H + 2 * g.ph) * ((int64_t)g.W + 2 * g.pw) * 4 + (int64_t)g.OH * g.OW * 8 + 4;
+}
+constexpr int64_t POOL_TILE_LDS = 60 * 1024;
+constexpr int POOL_TILE_ELEMS = 2048;
+
+// Whether the tile kernel takes the geometry; t's fields but vec if so.
+inline bool pool_tile_geometry(const PoolGeom& g, PoolTile& t, size_t& lds) {
+  const int64_t bytes = pool_tile_bytes(g);
+  const int64_t planes = g.N * g.C, hw = (int64_t)g.H * g.W;
+  if (g.ph > 4096 || g.pw > 4096 || bytes > POOL_TILE_LDS || hw * POOL_TILE_ELEMS > 0x7FFFFFFF)
+    return false;
+  // as many planes as make the workgroup's elements, unless that leaves the
+  // chip with fewer than four workgroups a CU
+  int64_t P = std::max<int64_t>(1, POOL_TILE_ELEMS / hw);
+  P = std::min<int64_t>(P, std::max<int64_t>(1, planes / (4 * (int64_t)device_cu_count())));
+  P = std::min<int64_t>(P, POOL_TILE_LDS / bytes);
+  // whole 4-element groups a workgroup
+  if (hw % 4 && P >= 4) P = P / 4 * 4;
+  t.g = g;
+  t.planes = planes;
+  t.P = (int)P;
+  t.rows4 = g.W % 4 == 0;
+  t.hp = g.H + 2 * g.ph;
+  t.wp = g.W + 2 * g.pw;
+  t.fd_hw = fast_div((uint32_t)hw);
+  t.fd_w = fast_div((uint32_t)g.W);
+  t.fd_pad = fast_div((uint32_t)(t.hp * t.wp));
+  t.fd_wp = fast_div((uint32_t)t.wp);
+  t.fd_win = fast_div((uint32_t)(g.OH * g.OW));
+  t.fd_ow = fast_div((uint32_t)g.OW);
+  t.fd_sh = fast_div((uint32_t)g.sh);
+  t.fd_sw = fast_div((uint32_t)g.sw);
+  lds = (size_t)(P * bytes);
+  return (planes + P - 1) / P <= 0x7FFFFFFF;
+}
+
+// Stages np padded planes from element e0 of x as fp32 bits.
+template <int XT>
+__device__ __forceinline__ void pool_stage(const uint8_t* __restrict__ x, int64_t e0, int np,
+                                           uint32_t* xt, const PoolTile& t) {
+  const PoolGeom& g = t.g;
+  const int hw = g.H * g.W, total = np * hw, pad = t.hp * t.wp;
+  auto at = [&](uint32_t e) {
+    const uint32_t p = fdiv(e, t.fd_hw), q = e - p * hw;
+    const uint32_t h = fdiv(q, t.fd_w), w = q - h * g.W;
+    return p * pad + (h + g.ph) * t.wp + w + g.pw;
+  };
+  if (t.vec) {
+    // two 4-element groups a lane in flight
+    for (int i = threadIdx.x * 4; i < total; i += 2048) {
+      xl_u32x4 v[2];
+      const bool two = i + 1024 < total;
+      v[0] = x4_raw<XT>(x, e0 + i);
+      if (two) v[1] = x4_raw<XT>(x, e0 + i + 1024);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        if (k && !two) break;
+        const uint32_t first = at((uint32_t)(i + 1024 * k));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          constexpr int B = XL<XT>::bits;
+          constexpr uint32_t mask = B == 32 ? 0xFFFFFFFFu : (1u << (B & 31)) - 1u;
+          const uint32_t word = v[k][q * B / 32];
+          const uint32_t d = t.rows4 ? first + q : at((uint32_t)(i + 1024 * k + q));
+          xt[d] = decode<XT>((word >> ((q * B) & 31)) & mask);
+        }
+      }
+    }
+  } else {
+    for (int i = threadIdx.x; i < total; i += 256) xt[at((uint32_t)i)] = decode<XT>(x_code<XT>(x, e0 + i));
+  }
+  if (g.ph | g.pw) {
+    for (int i = threadIdx.x; i < np * pad; i += 256) {
+      const uint32_t p = fdiv((uint32_t)i, t.fd_pad), q = (uint32_t)i - p * pad;
+      const int h = (int)fdiv(q, t.fd_wp) - g.ph, w = (int)q - (h + g.ph) * t.wp - g.pw;
+      if ((unsigned)h < (unsigned)g.H && (unsigned)w < (unsigned)g.W) continue;
+      const int hi = pad_index(h, g.H, g.pad_mode), wi = pad_index(w, g.W, g.pad_mode);
+      xt[i] = hi >= 0 && wi >= 0
+                  ? decode<XT>(x_code<XT>(x, e0 + (int64_t)p * hw + (int64_t)hi * g.W + wi))
+                  : 0u;  // the zero padding's +0
+    }
+  }
+}
+
+// Any geometry on planes that fit in LDS (pool_stage): first each window's
+// maximum and quotient grad / count, once a window, then each element adds the
+// shares of the windows holding it -- the sums, their order and every rounding
+// as max_pool2d_bwd_kernel's.  K, S: square windows of K and stride S fixed at
+// compile time (0: the geometry's), which takes the loops' bounds and the
+// divisions by the stride out (57.0 -> 49.8 us).  VALU-bound on the index
+// arithmetic; measured (256 x 64 planes of 28 x 28, fp32): 3 x 3 / 2 with
+// padding 49.8 us, 491 on max_pool2d_bwd_kernel's one-lane-an-element walk;
+// 3 x 3 / 1 88.1 us (1024).
+template <int XT, int K, int S>
+__global__ __launch_bounds__(256) void max_pool2d_bwd_tile_kernel(
+    const float* __restrict__ grad, const uint8_t* __restrict__ x, float* __restrict__ gi,
+    PoolTile t) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t pt_lds[];
+  const PoolGeom& g = t.g;
+  const int KH = K ? K : g.KH, KW = K ? K : g.KW, sh = S ? S : g.sh, sw = S ? S : g.sw;
+  auto div_h = [&](int v) { return S ? v / (S ? S : 1) : (int)fdiv((uint32_t)v, t.fd_sh); };
+  auto div_w = [&](int v) { return S ? v / (S ? S : 1) : (int)fdiv((uint32_t)v, t.fd_sw); };
+  const int64_t plane0 = (int64_t)blockIdx.x * t.P;
+  const int np = (int)min((int64_t)t.P, t.planes - plane0);
+  const int hw = g.H * g.W, npix = g.OH * g.OW, pad = t.hp * t.wp;
+  const float* xt = reinterpret_cast<const float*>(pt_lds);
+  // (maximum, quotient) of each window; 8-byte aligned
+  float2* win2 = reinterpret_cast<float2*>(pt_lds + ((t.P * pad + 1) & ~1));
+  const float* gp = grad + plane0 * npix;
+  // the first windows' grad is on its way while the planes are staged
+  float g0[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int o = threadIdx.x + 256 * k;
+    g0[k] = o < np * npix ? gp[o] : 0.0f;
+  }
+  pool_stage<XT>(x, plane0 * hw, np, pt_lds, t);
+  __syncthreads();
+  auto window = [&](int o, float gv) {
+    const uint32_t p = fdiv((uint32_t)o, t.fd_win), q = (uint32_t)o - p * npix;
+    const uint32_t i = fdiv(q, t.fd_ow), j = q - i * g.OW;
+    const float* win = xt + (p * t.hp + i * sh) * t.wp + j * sw;
+    float mx = -INFINITY;
+    int cnt = 0;
+    bool nan = false;
+    for (int kh = 0; kh < KH; ++kh)
+      for (int kw = 0; kw < KW; ++kw) {
+        const float v = win[kh * t.wp + kw];
+        nan |= isnan(v);
+        cnt = v > mx ? 1 : cnt + (v == mx);
+        mx = v > mx ? v : mx;
+      }
+    if (nan) mx = __builtin_nanf("");
+    if (nan || cnt == 0) cnt = 1;
+    win2[o] = make_float2(mx, gv / (float)cnt);
+  };
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if ((int)threadIdx.x + 256 * k < np * npix) window(threadIdx.x + 256 * k, g0[k]);
+  for (int o = threadIdx.x + 1024; o < np * npix; o += 256) window(o, gp[o]);
+  __syncthreads();
+  auto element = [&](int e) {
+    const uint32_t p = fdiv((uint32_t)e, t.fd_hw), q = (uint32_t)e - p * hw;
+    const int h = (int)fdiv(q, t.fd_w), w = (int)q - h * g.W;
+    const int hp = h + g.ph, wp = w + g.pw;
+    const float xv = xt[p * pad + hp * t.wp + wp];
+    // windows i with i*sh <= h + ph < i*sh + KH (and j likewise)
+    const int i0 = hp >= KH ? div_h((hp - KH)) + 1 : 0;
+    const int i1 = min(g.OH - 1, div_h(hp));
+    const int j0 = wp >= KW ? div_w((wp - KW)) + 1 : 0;
+    const int j1 = min(g.OW - 1, div_w(wp));
+    float sum = 0.0f;
+    for (int i = i0; i <= i1; ++i)
+      for (int j = j0; j <= j1; ++j) {
+        const float2 m = win2[(int)p * npix + i * g.OW + j];
+        sum += (xv == m.x ? 1.0f : 0.0f) * m.y;
+      }
+    return sum;
+  };
+  float* out = gi + plane0 * hw;
+  if (t.vec && t.rows4) {
+    // four neighbours of a row: their windows are walked once, each element
+    // adding those that hold it (in the same order as alone)
+    for (int e = threadIdx.x * 4; e < np * hw; e += 1024) {
+      const uint32_t p = fdiv((uint32_t)e, t.fd_hw), q = (uint32_t)e - p * hw;
+      const int h = (int)fdiv(q, t.fd_w), w = (int)q - h * g.W;
+      const int hp = h + g.ph, wp = w + g.pw;
+      const int i0 = hp >= KH ? div_h((hp - KH)) + 1 : 0;
+      const int i1 = min(g.OH - 1, div_h(hp));
+      const int j0 = wp >= KW ? div_w((wp - KW)) + 1 : 0;
+      const int j1 = min(g.OW - 1, div_w((wp + 3)));
+      float xv[4], sum[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        xv[k] = xt[p * pad + hp * t.wp + wp + k];
+        sum[k] = 0.0f;
+      }
+      for (int i = i0; i <= i1; ++i) {
+        const float2* row = win2 + (int)p * npix + i * g.OW;
+        for (int j = j0; j <= j1; ++j) {
+          const float2 m = row[j];
+          const int d = wp - j * sw;  // element k is the window's column d + k
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float v = sum[k] + (xv[k] == m.x ? 1.0f : 0.0f) * m.y;
+            sum[k] = (unsigned)(d + k) < (unsigned)KW ? v : sum[k];
+          }
+        }
+      }
+      *reinterpret_cast<float4*>(out + e) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+    }
+  } else if (t.vec) {
+    for (int e = threadIdx.x * 4; e < np * hw; e += 1024) {
+      float4 f;
+      f.x = element(e);
+      f.y = element(e + 1);
+      f.z = element(e + 2);
+      f.w = element(e + 3);
+      *reinterpret_cast<float4*>(out + e) = f;
+    }
+  } else {
+    for (int e = threadIdx.x; e < np * hw; e += 256) out[e] = element(e);
+  }
+}
+
 // 2 x 2 windows, stride 2, no padding, H and W even (every input element in
 // exactly one window: config [5]'s MaxPool2d(2, 2)): lane t makes window t's
 // four gradients, its two input rows read as 2-element loads and its two
@@ -753,6 +1032,22 @@ int launch_max_bwd(const float* grad, const void* x, float* gi, const PoolGeom& 
                        dim3(256), 0, stream, grad, xb, gi, g.W, g.OW,
                        fast_div((uint32_t)npix), fast_div((uint32_t)g.OW), (uint32_t)windows,
                        (uint32_t)npix);
+    return check_launch();
+  }
+  PoolTile t{};
+  size_t lds = 0;
+  if (pool_tile_geometry(g, t, lds)) {
+    t.vec = reinterpret_cast<uintptr_t>(x) % (4 * EB) == 0 &&
+            reinterpret_cast<uintptr_t>(gi) % 16 == 0 && (int64_t)t.P * g.H * g.W % 4 == 0 &&
+            g.N * g.C * g.H * (int64_t)g.W % 4 == 0;
+    const bool square = g.KH == g.KW && g.sh == g.sw;
+    auto kern = max_pool2d_bwd_tile_kernel<XT, 0, 0>;
+    if (square && g.KH == 3 && g.sh == 2) kern = max_pool2d_bwd_tile_kernel<XT, 3, 2>;
+    else if (square && g.KH == 3 && g.sh == 1) kern = max_pool2d_bwd_tile_kernel<XT, 3, 1>;
+    else if (square && g.KH == 3 && g.sh == 3) kern = max_pool2d_bwd_tile_kernel<XT, 3, 3>;
+    else if (square && g.KH == 2 && g.sh == 2) kern = max_pool2d_bwd_tile_kernel<XT, 2, 2>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((t.planes + t.P - 1) / t.P)), dim3(256), lds, stream,
+                       grad, xb, gi, t);
     return check_launch();
   }
   const int64_t blocks = (g.N * g.C * g.H * (int64_t)g.W + 255) / 256;
