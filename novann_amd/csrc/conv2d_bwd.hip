@@ -17,7 +17,7 @@
 //     codes permuted (exact).  With stride 1 and padding < kernel size,
 //     grad_input is the forward convolution of grad with Wf and zero padding
 //     (KH-1-ph, KW-1-pw), run by conv2d.hip's kernels;
-//   - dinput_direct_kernel: the sum above element by element in fp32, for the
+//   - dinput_phase_kernel: the sum above in fp32, one lane a pixel, for the
 //     other strides and paddings;
 //   - dweight_kernel: implicit GEMM on bf16 MFMA (v_mfma_f32_32x32x16_bf16):
 //     M = output channels (64 per workgroup), N = (c, kh, kw) (64 per
@@ -154,41 +154,136 @@ __global__ __launch_bounds__(256) void c1_tail_kernel(FinishArgs a, const float*
                           cg, (int)(b - a.wb - a.bb), t_lds);
 }
 
-// grad_input, one element per thread, fp32 accumulation over (kh, kw, co).
-template <int WT>
-__global__ __launch_bounds__(256) void dinput_direct_kernel(const float* __restrict__ grad,
-                                                           const uint8_t* __restrict__ w,
-                                                           const float* __restrict__ w_scale,
-                                                           float* __restrict__ gi, BwdGeom g) {
-  const int64_t total = (int64_t)g.N * g.C * g.H * g.W;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= total) return;
-  const int wx = (int)(t % g.W);
-  int64_t r = t / g.W;
-  const int hy = (int)(r % g.H);
-  r /= g.H;
-  const int c = (int)(r % g.C);
-  const int n = (int)(r / g.C);
+// grad_input for strides above 1 and wide paddings, in fp32: a lane makes one
+// input pixel of CT channels.  The taps that reach a pixel are those
+// congruent to its row and column modulo the strides, so a workgroup takes
+// pixels of one residue class (a phase) -- consecutive lanes on consecutive
+// output columns, all with the same taps -- and CT channels (a layer; the grid
+// is phases x layers x blocks of pixels).  Per tap and 128 output channels the
+// weights of those channels are decoded once into LDS, times the scale; a lane
+// then loads one grad value an output channel and adds CT products.  A tap
+// outside grad is skipped, not multiplied by zero.
+//
+// Bound by the LDS pipe (four broadcast reads to 16 products; two pixels a
+// lane need a select a product for the taps only one of them has: 271 us
+// against 181).  Where 256 pixels a workgroup would leave CUs idle (SPLIT) the
+// waves take a quarter of each stage's output channels of the same 64 pixels
+// and their sums are added in wave order.  Measured (E4M3, 64 <- 128 channels,
+// 3 x 3 / 2, 256 maps of 28 x 28): 181 us, 4414 with one lane an element that
+// decoded every weight for itself; 256 <- 256 channels, 8 maps of 7 x 7: 54.7
+// us (301; 147 without SPLIT).
+constexpr int DI_CO = 128;  // output channels a stage
+template <int WT, int CT, bool SPLIT>
+__global__ __launch_bounds__(256) void dinput_phase_kernel(const float* __restrict__ grad,
+                                                          const uint8_t* __restrict__ w,
+                                                          const float* __restrict__ w_scale,
+                                                          float* __restrict__ gi, BwdGeom g,
+                                                          int blocks, int layers) {
+  constexpr int LANES = SPLIT ? 64 : 256;  // lanes on different pixels
+  __shared__ __attribute__((aligned(16))) float wt[DI_CO * CT];
+  const int phase = (int)blockIdx.x / (blocks * layers), rest = (int)blockIdx.x - phase * blocks * layers;
+  const int layer = rest / blocks;
+  // pixels (h0 + sh i, w0 + sw j); taps a, a + sh, ... and b, b + sw, ...
+  const int h0 = phase / min(g.sw, g.W), w0 = phase - h0 * min(g.sw, g.W);
+  const int a = (h0 + g.ph) % g.sh, b = (w0 + g.pw) % g.sw;
+  const int Hp = (g.H - h0 + g.sh - 1) / g.sh, Wp = (g.W - w0 + g.sw - 1) / g.sw;
+  const int64_t total = (int64_t)g.N * Hp * Wp;
+  const int64_t first = (int64_t)(rest - layer * blocks) * LANES;
+  if (first >= total) return;  // the whole workgroup
+  const int wave = SPLIT ? threadIdx.x >> 6 : 0;
+  const int px = SPLIT ? threadIdx.x & 63 : threadIdx.x;
+  const int64_t q = first + px;
+  const bool live = q < total;
+  const int64_t n = live ? q / ((int64_t)Hp * Wp) : 0;
+  const int r = live ? (int)(q - n * Hp * Wp) : 0;
+  const int i = r / Wp, h = h0 + g.sh * i, x = w0 + g.sw * (r - i * Wp);
+  const int c0 = layer * CT;
   const float s = w_scale ? *w_scale : 1.0f;
-  float acc = 0.0f;
-  for (int kh = 0; kh < g.KH; ++kh) {
-    const int th = hy + g.ph - kh;
-    if (th < 0 || th % g.sh) continue;
-    const int oh = th / g.sh;
-    if (oh >= g.OH) continue;
-    for (int kw = 0; kw < g.KW; ++kw) {
-      const int tw = wx + g.pw - kw;
-      if (tw < 0 || tw % g.sw) continue;
-      const int ow = tw / g.sw;
-      if (ow >= g.OW) continue;
-      for (int co = 0; co < g.C_out; ++co) {
-        const float gv = grad[(((int64_t)n * g.C_out + co) * g.OH + oh) * g.OW + ow];
-        const int64_t e = (((int64_t)co * g.C + c) * g.KH + kh) * g.KW + kw;
-        acc += u2f(decode<WT>(code_at<WT>(w, e))) * s * gv;
+  float acc[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) acc[c] = 0.0f;
+
+  constexpr int NL = DI_CO * CT / 256;  // weights a lane stages
+  const int kk = g.KH * g.KW;
+  uint32_t code[NL];
+  // codes of stage (tap kh, kw; output channels from co0): channel fastest
+  auto fetch = [&](int kh, int kw, int co0) {
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      const int e = threadIdx.x + 256 * k, co = co0 + e / CT, c = c0 + e % CT;
+      code[k] = 0;
+      if (co < g.C_out && c < g.C)
+        code[k] = code_at<WT>(w, ((int64_t)co * g.C + c) * kk + kh * g.KW + kw);
+    }
+  };
+  const int64_t plane = (int64_t)g.OH * g.OW;
+  int kh = a, kw = b, co0 = 0;
+  if (kh < g.KH && kw < g.KW) fetch(kh, kw, co0);
+  while (kh < g.KH && kw < g.KW) {
+    __syncthreads();  // the previous stage is done with
+#pragma unroll
+    for (int k = 0; k < NL; ++k) wt[threadIdx.x + 256 * k] = u2f(decode<WT>(code[k])) * s;
+    __syncthreads();
+    const int tkh = kh, tkw = kw, tco = co0, nco = min(DI_CO, g.C_out - co0);
+    // the next stage's codes are on their way while this one multiplies
+    co0 += DI_CO;
+    if (co0 >= g.C_out) {
+      co0 = 0;
+      kw += g.sw;
+      if (kw >= g.KW) {
+        kw = b;
+        kh += g.sh;
       }
     }
+    if (kh < g.KH) fetch(kh, kw, co0);
+    const int dh = h + g.ph - tkh, dw = x + g.pw - tkw;  // multiples of the strides
+    const int oh = dh / g.sh, ow = dw / g.sw;
+    if (live && dh >= 0 && dw >= 0 && oh < g.OH && ow < g.OW) {
+      const float* gp = grad + ((n * g.C_out + tco) * g.OH + oh) * g.OW + ow;
+      auto add = [&](float gv, int co) {
+#pragma unroll
+        for (int c = 0; c < CT; c += 4) {
+          const float4 v = *reinterpret_cast<const float4*>(wt + co * CT + c);
+          acc[c] = __builtin_fmaf(v.x, gv, acc[c]);
+          acc[c + 1] = __builtin_fmaf(v.y, gv, acc[c + 1]);
+          acc[c + 2] = __builtin_fmaf(v.z, gv, acc[c + 2]);
+          acc[c + 3] = __builtin_fmaf(v.w, gv, acc[c + 3]);
+        }
+      };
+      int co = SPLIT ? nco * wave / 4 : 0;
+      const int to = SPLIT ? nco * (wave + 1) / 4 : nco;
+      for (; co + 8 <= to; co += 8) {
+        float gv[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) gv[k] = gp[(co + k) * plane];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) add(gv[k], co + k);
+      }
+      for (; co < to; ++co) add(gp[co * plane], co);
+    }
   }
-  gi[t] = acc;
+  if constexpr (SPLIT) {
+    // the quarters added in wave order, 4 channels of LDS at a time
+    static_assert(DI_CO * CT >= 256 * 4, "LDS of the sums");
+#pragma unroll
+    for (int c = 0; c < CT; c += 4) {
+      __syncthreads();
+      *reinterpret_cast<float4*>(wt + 4 * threadIdx.x) =
+          make_float4(acc[c], acc[c + 1], acc[c + 2], acc[c + 3]);
+      __syncthreads();
+      if (wave == 0) {
+#pragma unroll
+        for (int k = 1; k < 4; ++k)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[c + e] += wt[4 * (64 * k + px) + e];
+      }
+    }
+    if (wave) return;
+  }
+  if (!live) return;
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+    if (c0 + c < g.C) gi[((n * g.C + c0 + c) * g.H + h) * g.W + x] = acc[c];
 }
 
 constexpr int DW_THREADS = 256;
@@ -1147,11 +1242,21 @@ int launch_dinput(const float* grad, const void* w, const void* wf, const float*
                                  gi, stream);
     if (rc != NOVAQ_ENOTSUP) return rc;
   }
-  const int64_t total = (int64_t)g.N * g.C * g.H * g.W;
-  const int64_t blocks = (total + 255) / 256;
-  if (blocks > 0x7FFFFFFF) return NOVAQ_EINVAL;
-  hipLaunchKernelGGL(dinput_direct_kernel<WT>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                     grad, static_cast<const uint8_t*>(w), w_scale, gi, g);
+  // the blocks of the largest phase; 16 channels a layer, 8 for the few of a
+  // first layer
+  const int64_t pixels = (int64_t)g.N * ((g.H + (int64_t)g.sh - 1) / g.sh) * ((g.W + (int64_t)g.sw - 1) / g.sw);
+  const int64_t phases = (int64_t)std::min(g.sh, g.H) * std::min(g.sw, g.W);
+  const int ct = g.C > 8 ? 16 : 8;
+  const int64_t layers = (g.C + ct - 1) / ct;
+  // 256 pixels a workgroup while that gives every CU four workgroups
+  const bool split = (pixels + 255) / 256 * layers * phases < 4 * (int64_t)device_cu_count();
+  const int64_t per = split ? 64 : 256, blocks = (pixels + per - 1) / per;
+  if (blocks > 0x7FFFFFFF || blocks * layers > 0x7FFFFFFF || blocks * layers * phases > 0x7FFFFFFF)
+    return NOVAQ_EINVAL;
+  auto kern = split ? (ct == 16 ? dinput_phase_kernel<WT, 16, true> : dinput_phase_kernel<WT, 8, true>)
+                    : (ct == 16 ? dinput_phase_kernel<WT, 16, false> : dinput_phase_kernel<WT, 8, false>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(blocks * layers * phases)), dim3(256), 0, stream, grad,
+                     static_cast<const uint8_t*>(w), w_scale, gi, g, (int)blocks, (int)layers);
   return check_launch();
 }
 
