@@ -37,6 +37,7 @@
 
 #include <algorithm>
 
+#include "conv2d_chunk.h"
 #include "conv2d_gather.h"
 #include "novaq_convert.h"
 #include "novaq_epilogue.h"
@@ -1633,6 +1634,23 @@ bool launch_smallc(const uint8_t* x, const float* x_scale, const void* w, const 
   return true;
 }
 
+// The chunked path where it takes the shape with at least `least` workgroups;
+// returns false otherwise.
+template <int WT, int XT>
+bool launch_chunk(const uint8_t* x, const float* x_scale, const void* w, const float* w_scale,
+                  const Epilogue& ep, void* y, const ConvGeom& cg, int least, hipStream_t stream,
+                  int* rc) {
+  if ((cg.pad_mode != NOVAQ_PAD_ZEROS && (cg.ph || cg.pw)) || cg.KH != cg.KW ||
+      (cg.KH != 3 && cg.KH != 1) || cg.C % CK_C)
+    return false;
+  ChunkGeom g{};
+  g.N = cg.N; g.C = cg.C; g.H = cg.H; g.W = cg.W; g.M = cg.C_out; g.KH = cg.KH; g.KW = cg.KW;
+  g.sh = cg.sh; g.sw = cg.sw; g.ph = cg.ph; g.pw = cg.pw; g.OH = cg.OH; g.OW = cg.OW;
+  const auto* wq = static_cast<const uint8_t*>(w);
+  return cg.KH == 3 ? chunk_launch<WT, XT, 9>(x, x_scale, wq, w_scale, ep, y, g, least, stream, rc)
+                    : chunk_launch<WT, XT, 1>(x, x_scale, wq, w_scale, ep, y, g, least, stream, rc);
+}
+
 // The gathered path where it takes the shape; returns false otherwise.
 template <int WT, int XT>
 bool launch_gather(const uint8_t* x, const float* x_scale, const void* w, const float* w_scale,
@@ -1677,6 +1695,20 @@ int launch(const uint8_t* x, const float* x_scale, const void* w, const float* w
   int ipt = 0;
   const bool band = band_geometry<WT>(g, b, band_lds, &ipt, ep.out_dtype);
   const int64_t co_blocks = (g.C_out + CO_TILE - 1) / CO_TILE;
+  // The chunked path where its workgroups cover an eighth of the CUs (96 -> 70
+  // channels, 3 maps of 13 x 17 = 12 workgroups: 17.1 us, gathered 13.2; 64 ->
+  // 64, 16 maps of 14 x 14 = 32: 9.8 against 10.9), but for one chunk of FP4
+  // weights on bands that fill the chip (32 -> 64, 256 maps of 28 x 28: 25.0
+  // us, in bands 23.5).
+  if constexpr (dtype_bits(WT) <= 8) {
+    const bool bands_best = WT == E2M1 && band && band_lds <= BAND_LDS_FOUR && g.C == CK_C &&
+                            b.taps == 9 && g.sh == 1 && g.sw == 1 &&
+                            (int64_t)g.N * b.bands * co_blocks >= 2 * (int64_t)device_cu_count();
+    int rc = NOVAQ_OK;
+    if (!bands_best &&
+        launch_chunk<WT, XT>(x, x_scale, w, w_scale, ep, y, g, device_cu_count() / 8, stream, &rc))
+      return rc;
+  }
   // The gathered path wherever no band fits in LDS, and where bands would
   // leave CUs idle (64 -> 64 channels, 3 x 3, 16 maps of 14 x 14 = 16 bands:
   // 11.2 us gathered, 23.1 in bands; 400 bands of 16 -> 48 channels 28.6
