@@ -100,7 +100,7 @@ class AdamW:
             is_bn_param = getattr(p, "name", None) in ("gamma", "beta")
             hp = _lib.AdamW(self.lr, self.b1, self.b2, self.eps, self.wd, self.t,
                             0 if is_bn_param else 1)
-            stream = torch.cuda.current_stream(w.device).cuda_stream
+            stream = torch._C._cuda_getCurrentRawStream(w.get_device())
             if w.dtype == torch.float64:
                 g, g32 = _dev_grad64(p.grad, w.device)
                 if g.numel() != w.numel():

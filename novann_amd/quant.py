@@ -53,7 +53,8 @@ def _require_holds(t: torch.Tensor, dtype: str, n: int, what: str) -> None:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # (the address alone: building a torch Stream costs 1.9 us a call, this 0.1)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _require_device(t: torch.Tensor, what: str) -> None:
