@@ -16,9 +16,9 @@
 // epilogue in 4-element runs along n.
 //
 // Each operand comes in one of two layouts:
-//   row: K contiguous.  In block k0, lane (r, g) (r = lane % 16, g = lane / 16)
-//        loads the 16 consecutive elements k0 + 16 g .. + 15 of row 16 t + r
-//        for tile t: two MFMA steps of 8.
+//   row: K contiguous (long products: LsQuad instead).  In block k0, lane (r, g)
+//        (r = lane % 16, g = lane / 16) loads the 16 consecutive elements
+//        k0 + 16 g .. + 15 of row 16 t + r for tile t: two MFMA steps of 8.
 //   col: K-major (element (k, m) at k * pitch + m).  The lane loads, for each
 //        of the same 16 k, the T consecutive elements T r .. T r + T - 1 (T
 //        tiles): element t of every run makes tile t's fragment, so tile t
@@ -29,18 +29,23 @@
 // the last block, when K % 64 != 0, is loaded element by element with zeros
 // past K, and indices past M or N are clamped to the last one (never stored).
 //
-// What bounds it: a CU's load rate (about 94 GB/s of 16-byte loads) times the
-// operand bytes of a tile, then latency; so the tile is 64 x 64 (4 waves, two
-// workgroups a CU) when those tiles cover the CUs, 32 x 32 on 8 waves below
-// that, and 16 x 16 on 16 waves for at most 16 rows (every CU then streams its
-// own 16 rows of W).  Measured (E4M3 W 4096 x 4096, fp32 x, warm MALL; the
-// guarded 128 x 256-tile kernel it replaced in brackets): 1 row 6.8 us (296),
-// 16 rows 12.0 (306), 64 rows 21.8 (342); 500 x 1024 x 1024 13.0 (120); 333 x
-// 777 x 1111 16.9 (277).
+// What bounds it: a CU's load rate times the operand bytes of a tile, then
+// latency; so the tile is 64 x 64 (4 waves, two workgroups a CU) when those
+// tiles cover the CUs, 32 x 32 on 8 waves below that, and 16 x 16 on 16 waves
+// for at most 16 rows (every CU then streams its own 16 rows of W).  A fragment
+// load straight from 16 rows reaches a line a lane and the CU only 94 GB/s of
+// them, whatever the depth of the pipeline (2 to 8 half blocks in flight: the
+// same time); row operands of long products are therefore read as LsQuad says.
+// Measured (E4M3 W 4096 x 4096, fp32 x, warm MALL; the guarded 128 x 256-tile
+// kernel it replaced in brackets): 1 row 6.8 us (296), 16 rows 8.4 (306), 64
+// rows 15.7 (342), 14.6 with FP4 W, 9.6 with bf16 x too; 500 x 1024 x 1024 12.6
+// (120); 333 x 777 x 1111 16.8 (277).
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "novaq_convert.h"
 #include "novaq_epilogue.h"
@@ -206,6 +211,88 @@ struct LsRow {
   __device__ __forceinline__ int index(const int t, int r) const { return 16 * t + r; }
 };
 
+// Row operand of a small tile, read 64 contiguous bytes a quad of lanes: a
+// memory instruction costs about a cycle per line and quad, and LsRow's lanes
+// are each on a row of their own.  In block k0 (LQ_KB elements), lane (h, m, c)
+// = (lane / 16, lane / 4 % 4, lane % 4) loads, for j = 0 .. 3, chunk c of K
+// quarter h of row 4 m + j; a 4 x 4 transpose within each quad (two rounds of
+// lane exchanges) then gives it the four chunks of row 4 m + c = lane % 16, the
+// fragments' row.  Fragment step s holds elements k0 + 32 h + 8 s .. + 7.
+constexpr int LQ_KB = 128;
+
+template <int DT, int T>
+struct LsQuad {
+  static constexpr int bits = dtype_bits(DT);
+  static constexpr int QB = 32 * bits / 8;              // bytes of a K quarter
+  static constexpr int GROUPS = QB > 64 ? QB / 64 : 1;  // loads of 4 chunks a block
+  static constexpr int CB = QB / GROUPS / 4;            // bytes of a chunk
+  static constexpr int CW = CB / 4;                     // words
+  static constexpr int STEPS = 4 / GROUPS;              // steps a group
+  typedef uint32_t Chunk __attribute__((ext_vector_type(CW)));
+  struct Regs {
+    Chunk w[T][4];
+  };
+  const uint8_t* row[T][4];
+  bool odd, high;
+
+  __device__ __forceinline__ void init(const uint8_t* p, int64_t pitch, int i0, int count, int lane) {
+    odd = lane & 1;
+    high = lane & 2;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        row[t][j] = p + (int64_t)min(i0 + 16 * t + (lane >> 2 & 3) * 4 + j, count - 1) * pitch +
+                    (lane >> 4) * QB + (lane & 3) * CB;
+  }
+  __device__ __forceinline__ void load(Regs& r, int k0, const int group) const {
+    const int64_t b = (int64_t)k0 * bits / 8 + group * 4 * CB;
+    typedef Chunk ChunkU __attribute__((aligned(1)));
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r.w[t][j] = *reinterpret_cast<const ChunkU*>(row[t][j] + b);
+  }
+  template <int CTRL>
+  static __device__ __forceinline__ uint32_t quad(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+  }
+  // chunk j of load k <-> chunk k of load j, across the lanes of a quad
+  __device__ __forceinline__ void turn(Regs& r) const {
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int i = 0; i < CW; ++i) {
+        uint32_t a[4], b[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = r.w[t][j][i];
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {  // lanes c, c ^ 1
+          const uint32_t p = quad<0xB1>(a[j + 1]), q = quad<0xB1>(a[j]);
+          b[j] = odd ? p : a[j];
+          b[j + 1] = odd ? a[j + 1] : q;
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {     // lanes c, c ^ 2
+          const uint32_t p = quad<0x4E>(b[j + 2]), q = quad<0x4E>(b[j]);
+          r.w[t][j][i] = high ? p : b[j];
+          r.w[t][j + 2][i] = high ? b[j + 2] : q;
+        }
+      }
+  }
+  // tile t's fragment of step s (turned)
+  static __device__ __forceinline__ ls_bf16x8 frag(const Regs& r, const int t, const int s) {
+    constexpr int N8 = bits / 4;  // words of 8 elements
+    uint32_t w[N8];
+#pragma unroll
+    for (int i = 0; i < N8; ++i) {
+      const int at = (s % STEPS) * N8 + i;
+      w[i] = r.w[t][at / CW][at % CW];
+    }
+    return ls_decode8<DT>(w);
+  }
+};
+
 // Col operand: T tiles, element (k, i) at row k of `pitch` bytes.
 template <int DT, int T>
 struct LsCol {
@@ -308,7 +395,7 @@ struct SplitGeom {
 
 // x_sum (XCOL, fp32): x_sum[m] = sum over k of X(m, k) in fp32, made by the
 // workgroups of the first tile column.
-template <int XT, bool XCOL, int WT, bool WCOL, int MT, int NT, int NWV>
+template <int XT, bool XCOL, int WT, bool WCOL, int MT, int NT, int NWV, bool QUAD>
 __global__ __launch_bounds__(NWV * 64) void linear_split_kernel(
     const uint8_t* __restrict__ x, const float* __restrict__ x_scale,
     const uint8_t* __restrict__ w, const float* __restrict__ w_scale, Epilogue ep,
@@ -349,8 +436,11 @@ __global__ __launch_bounds__(NWV * 64) void linear_split_kernel(
   for (int i = 0; i < MT; ++i) xs[i] = 0.0f;
   const bool sums = XCOL && x_sum && n0 == 0;
 
-  const int whole = g.K / LS_KB, blocks = whole + (g.K % LS_KB != 0);
+  // blocks of this kernel's size; what is left of K goes 64 at a time
+  constexpr int KB = QUAD ? LQ_KB : LS_KB;
+  const int whole = g.K / KB, blocks = whole + (g.K % KB != 0);
   const int b0 = (int)((int64_t)blocks * wave / NWV), b1 = (int)((int64_t)blocks * (wave + 1) / NWV);
+  const int e = min(b1, whole);
   // One MFMA step: half u of a block.
   auto multiply = [&](const typename X::Regs& rx, const typename Wt::Regs& rw, const int u) {
     ls_bf16x8 a[NT];
@@ -370,37 +460,103 @@ __global__ __launch_bounds__(NWV * 64) void linear_split_kernel(
       }
     }
   };
-  // Two register sets an operand, the next one's loads in flight while a step
-  // multiplies: half blocks alternate by step, whole blocks by block.
-  typename X::Regs rx[2];
-  typename Wt::Regs rw[2];
-  const int e = min(b1, whole);
-  // Block b, whose first half (and whole codes, in set P) is loaded already.
-  auto block = [&](int b, const int P) {
-    if constexpr (X::HALF) xo.load(rx[1], b * LS_KB, 1);
-    if constexpr (Wt::HALF) wo.load(rw[1], b * LS_KB, 1);
-    multiply(rx[X::HALF ? 0 : P], rw[Wt::HALF ? 0 : P], 0);
-    if (b + 1 < e) {
-      xo.load(rx[X::HALF ? 0 : P ^ 1], (b + 1) * LS_KB, 0);
-      wo.load(rw[Wt::HALF ? 0 : P ^ 1], (b + 1) * LS_KB, 0);
-    }
-    multiply(rx[X::HALF ? 1 : P], rw[Wt::HALF ? 1 : P], 1);
-  };
-  if (b0 < e) {
-    xo.load(rx[0], b0 * LS_KB, 0);
-    wo.load(rw[0], b0 * LS_KB, 0);
-  }
-  for (int b = b0; b < e; b += 2) {
-    block(b, 0);
-    if (b + 1 < e) block(b + 1, 1);
-  }
-  if (b1 > whole && b0 < b1) {  // this wave has the ragged last block
+  // the last K elements from k0, fewer than a 64-K block
+  auto tail = [&](typename X::Regs& rx, typename Wt::Regs& rw, int k0) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      if (u == 0 || X::HALF) xo.load_tail(rx[0], whole * LS_KB, u, g.K);
-      if (u == 0 || Wt::HALF) wo.load_tail(rw[0], whole * LS_KB, u, g.K);
-      multiply(rx[0], rw[0], u);
+      if (u == 0 || X::HALF) xo.load_tail(rx, k0, u, g.K);
+      if (u == 0 || Wt::HALF) wo.load_tail(rw, k0, u, g.K);
+      multiply(rx, rw, u);
     }
+  };
+  const bool ragged = b1 > whole && b0 < b1;  // this wave has the ragged last block
+  // Two register sets an operand, the next one's loads in flight while a step
+  // multiplies.
+  if constexpr (QUAD) {
+    using Q = LsQuad<XT, MT>;
+    using R = LsQuad<WT, NT>;
+    Q xq;
+    R wq;
+    xq.init(x, g.x_pitch, m0, g.M, lane);
+    wq.init(w, g.w_pitch, n0, g.N, lane);
+    typename Q::Regs qx[2];
+    typename R::Regs qw[2];
+    static_assert(R::GROUPS == 1, "weights of 16 bits and fewer");
+    // Block b, whose first x group (and whole block, in set P) is loaded already.
+    auto block = [&](int b, const int P) {
+      const bool next = b + 1 < e;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int px = Q::GROUPS == 2 ? s >> 1 : P;
+        if constexpr (Q::GROUPS == 2) {
+          if (s == 0) xq.load(qx[1], b * LQ_KB, 1);
+          if (s == 2 && next) xq.load(qx[0], (b + 1) * LQ_KB, 0);
+        } else {
+          if (s == 0 && next) xq.load(qx[P ^ 1], (b + 1) * LQ_KB, 0);
+        }
+        if (s == 0) {
+          if (next) wq.load(qw[P ^ 1], (b + 1) * LQ_KB, 0);
+          wq.turn(qw[P]);
+        }
+        if (s % Q::STEPS == 0) xq.turn(qx[px]);
+        ls_bf16x8 a[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) a[j] = R::frag(qw[P], j, s);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const ls_bf16x8 v = Q::frag(qx[px], i, s);
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j], v, acc[i][j], 0, 0, 0);
+        }
+      }
+    };
+    if (b0 < e) {
+      xq.load(qx[0], b0 * LQ_KB, 0);
+      wq.load(qw[0], b0 * LQ_KB, 0);
+    }
+    for (int b = b0; b < e; b += 2) {
+      block(b, 0);
+      if (b + 1 < e) block(b + 1, 1);
+    }
+    if (ragged) {
+      typename X::Regs rx;
+      typename Wt::Regs rw;
+      int k0 = whole * LQ_KB;
+      if (k0 + LS_KB <= g.K) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          if (u == 0 || X::HALF) xo.load(rx, k0, u);
+          if (u == 0 || Wt::HALF) wo.load(rw, k0, u);
+          multiply(rx, rw, u);
+        }
+        k0 += LS_KB;
+      }
+      if (k0 < g.K) tail(rx, rw, k0);
+    }
+  } else {
+    typename X::Regs rx[2];
+    typename Wt::Regs rw[2];
+    // Block b, whose first half (and whole codes, in set P) is loaded already.
+    auto block = [&](int b, const int P) {
+      if constexpr (X::HALF) xo.load(rx[1], b * LS_KB, 1);
+      if constexpr (Wt::HALF) wo.load(rw[1], b * LS_KB, 1);
+      multiply(rx[X::HALF ? 0 : P], rw[Wt::HALF ? 0 : P], 0);
+      if (b + 1 < e) {
+        xo.load(rx[X::HALF ? 0 : P ^ 1], (b + 1) * LS_KB, 0);
+        wo.load(rw[Wt::HALF ? 0 : P ^ 1], (b + 1) * LS_KB, 0);
+      }
+      multiply(rx[X::HALF ? 1 : P], rw[Wt::HALF ? 1 : P], 1);
+    };
+    if (b0 < e) {
+      xo.load(rx[0], b0 * LS_KB, 0);
+      wo.load(rw[0], b0 * LS_KB, 0);
+    }
+    for (int b = b0; b < e; b += 2) {
+      block(b, 0);
+      if (b + 1 < e) block(b + 1, 1);
+    }
+    if (ragged) tail(rx[0], rw[0], whole * LS_KB);
   }
 
   // add the waves' tiles in wave order, 16 rows of X (one MT tile) at a time
@@ -474,7 +630,7 @@ __global__ __launch_bounds__(NWV * 64) void linear_split_kernel(
   }
 }
 
-template <int XT, bool XCOL, int WT, bool WCOL, int MT, int NT, int NWV>
+template <int XT, bool XCOL, int WT, bool WCOL, int MT, int NT, int NWV, bool QUAD = false>
 int split_launch_tile(const uint8_t* x, const float* x_scale, const uint8_t* w,
                       const float* w_scale, const Epilogue& ep, void* y, float* x_sum,
                       SplitGeom g, hipStream_t stream) {
@@ -483,7 +639,7 @@ int split_launch_tile(const uint8_t* x, const float* x_scale, const uint8_t* w,
   if (tm * tn > 0x7FFFFFFF) return NOVAQ_EINVAL;
   g.tiles_m = (int)tm;
   g.tiles_n = (int)tn;
-  hipLaunchKernelGGL((linear_split_kernel<XT, XCOL, WT, WCOL, MT, NT, NWV>),
+  hipLaunchKernelGGL((linear_split_kernel<XT, XCOL, WT, WCOL, MT, NT, NWV, QUAD>),
                      dim3((unsigned)(tm * tn)), dim3(NWV * 64), 0, stream, x, x_scale, w, w_scale,
                      ep, y, x_sum, g);
   return check_launch();
@@ -505,6 +661,21 @@ int split_launch(const uint8_t* x, const float* x_scale, int64_t M, int64_t K, c
   g.n_vec = N % 4 == 0;
   const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
   if constexpr (!XCOL && !WCOL) {
+    // Lines read whole by quads of lanes (LsQuad) halve a long product's time
+    // (64 x 4096 x 4096, bf16 x, FP4 W: 9.6 us against 14.7).  Its larger blocks
+    // and registers need waves with work for them: from 4 rows (2 rows 7.5 us
+    // against 7.3), 2048 K over 16 waves (1024: 5.0, 4.5), and with one
+    // workgroup a CU 512 K over 8 (128 x 256 x 256: 5.5, 4.8; 64 x 2048 x 513:
+    // 6.0, 8.3), with more 1024 K without a rest (1000 x 500 x 784: 15.2, 11.4;
+    // 500 x 1024 x 1024: 8.9, 9.4) or 2048.
+    if constexpr (dtype_bits(WT) <= 16) {
+      const int64_t tiles32 = ((M + 31) / 32) * ((N + 31) / 32);
+      if (M >= 4 && M <= 16 && K >= 2048)
+        return split_launch_tile<XT, XCOL, WT, WCOL, 1, 1, 16, true>(x, x_scale, w, w_scale, ep, y, x_sum, g, stream);
+      if (M > 16 && tiles64 < device_cu_count() &&
+          (K >= 2048 || (tiles32 <= device_cu_count() ? K >= 512 : K >= 1024 && K % LQ_KB == 0)))
+        return split_launch_tile<XT, XCOL, WT, WCOL, 2, 2, 8, true>(x, x_scale, w, w_scale, ep, y, x_sum, g, stream);
+    }
     if (M <= 16)
       return split_launch_tile<XT, XCOL, WT, WCOL, 1, 1, 16>(x, x_scale, w, w_scale, ep, y, x_sum, g, stream);
   }
