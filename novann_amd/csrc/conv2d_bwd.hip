@@ -106,14 +106,25 @@ struct FinishArgs {
 };
 
 // COLS: the column sums' block width (16 for the one-input-channel kernel's
-// many short partials, else 64).
+// many short partials, 256 = four columns a lane for many columns, else 64).
 template <int WT, int COLS>
 __global__ __launch_bounds__(1024) void finish_kernel(FinishArgs a, int C_out, int C, int KH,
                                                       int KW) {
-  constexpr int SLICES = 1024 / COLS;
-  __shared__ float part[SLICES][COLS];
+  constexpr bool QUADS = COLS == CSQ_COLS;
+  constexpr int SLICES = QUADS ? CS_SLICES : 1024 / COLS;
+  __shared__ __attribute__((aligned(16))) float part[SLICES][COLS];
   const unsigned b = blockIdx.x;
-  if (b < a.wb) {
+  if constexpr (QUADS) {
+    if (b < a.wb) {
+      colsum_quads(a.part, a.rows, a.wcols, a.gw, a.pt, a.pco, a.pc, b, part);
+    } else if (b < a.wb + a.bb) {
+      colsum_block(a.bpart, a.rows, a.bcols, a.gb, 0, 0, 0, b - a.wb,
+                   reinterpret_cast<float(*)[CS_COLS]>(&part[0][0]));
+    } else {
+      const int64_t t = (int64_t)(b - a.wb - a.bb) * 1024 + threadIdx.x;
+      if (t < a.flip_items) flip_item<WT>(a.w, a.wf, t, C_out, C, KH, KW);
+    }
+  } else if (b < a.wb) {
     colsum_block<COLS, SLICES>(a.part, a.rows, a.wcols, a.gw, a.pt, a.pco, a.pc, b, part);
   } else if (b < a.wb + a.bb) {
     colsum_block<COLS, SLICES>(a.bpart, a.rows, a.bcols, a.gb, 0, 0, 0, b - a.wb, part);
@@ -920,8 +931,7 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
 
 constexpr int DR_MAX_XJ = 5;
 
-// grad_weight and grad_bias of a one-input-channel convolution (config [5]'s
-// first layer), stride 1, at most 16 window taps: as a GEMM, M = the output
+// grad_weight and grad_bias of a one-input-channel convolution, stride 1, at most 16 window taps: as a GEMM, M = the output
 // channels, N = the taps, K = the output pixels, so v_mfma_f32_16x16x32_bf16
 // tiles fill (the general kernel's N = (c, kh, kw) would hold 9 of 64
 // columns).  A unit is a band of RB output rows of one image; a workgroup
@@ -1174,7 +1184,8 @@ int64_t flip_items(const BwdGeom& g, int wt) {
 
 template <int COLS>
 int launch_finish_cols(FinishArgs a, int wt, const BwdGeom& g, hipStream_t stream) {
-  const int64_t wb = (a.wcols + COLS - 1) / COLS, bb = (a.bcols + COLS - 1) / COLS;
+  constexpr int BCOLS = COLS == CSQ_COLS ? CS_COLS : COLS;
+  const int64_t wb = (a.wcols + COLS - 1) / COLS, bb = (a.bcols + BCOLS - 1) / BCOLS;
   const int64_t fb = (a.flip_items + 1023) / 1024;
   const int64_t blocks = wb + bb + fb;
   if (blocks == 0) return NOVAQ_OK;
@@ -1196,8 +1207,13 @@ int launch_finish_cols(FinishArgs a, int wt, const BwdGeom& g, hipStream_t strea
 
 // With one input channel (C == 1: the one-input-channel kernel's up to
 // D1_CHUNKS partials of C_out x taps columns) the sums take 16 columns a
-// workgroup, otherwise 64.
+// workgroup; with columns for one workgroup of 256 a CU, four a lane; otherwise
+// 64 (18432 columns: 72 workgroups of 256 would read the partials on a quarter
+// of the CUs).
 int launch_finish(FinishArgs a, int wt, const BwdGeom& g, hipStream_t stream) {
+  if (g.C > 1 && a.wcols % 4 == 0 && a.wcols >= (int64_t)CSQ_COLS * device_cu_count() &&
+      a.wcols <= 0x7FFFFFFF)
+    return launch_finish_cols<CSQ_COLS>(a, wt, g, stream);
   return g.C == 1 ? launch_finish_cols<16>(a, wt, g, stream) : launch_finish_cols<64>(a, wt, g, stream);
 }
 

@@ -63,4 +63,51 @@ __device__ inline void colsum_block(const float* __restrict__ x, int64_t rows, i
   }
 }
 
+typedef float cs_f32x4 __attribute__((ext_vector_type(4)));
+
+// The same sums bit for bit with four consecutive columns a lane: 256 columns
+// a workgroup of 1024 lanes over 16 slices, for column counts that still fill
+// the chip with a quarter of the workgroups, each load and wait serving four
+// columns.  cols a multiple of 4 below 2^31, x on 16 bytes.  Measured (32 rows
+// of 147456 columns, permuted): 9.2 us with a column a lane, 6.1 here.
+constexpr int CSQ_COLS = 256;
+
+__device__ inline void colsum_quads(const float* __restrict__ x, int64_t rows, int64_t cols,
+                                    float* __restrict__ out, int pt, int pco, int pc, int64_t blk,
+                                    float (*part)[CSQ_COLS]) {
+  const int tx = threadIdx.x % 64, ty = threadIdx.x / 64;
+  const int64_t c = blk * CSQ_COLS + 4 * tx;
+  const int64_t per = (rows + CS_SLICES - 1) / CS_SLICES;
+  const int64_t rb = ty * per, re = min(rows, rb + per);
+  cs_f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (c < cols) {
+    cs_f32x4 a0 = s, a1 = s, a2 = s, a3 = s;
+    const float* p = x + c;
+    int64_t r = rb;
+#pragma unroll 2
+    for (; r + 3 < re; r += 4) {
+      a0 += *reinterpret_cast<const cs_f32x4*>(p + r * cols);
+      a1 += *reinterpret_cast<const cs_f32x4*>(p + (r + 1) * cols);
+      a2 += *reinterpret_cast<const cs_f32x4*>(p + (r + 2) * cols);
+      a3 += *reinterpret_cast<const cs_f32x4*>(p + (r + 3) * cols);
+    }
+    for (; r < re; ++r) a0 += *reinterpret_cast<const cs_f32x4*>(p + r * cols);
+    s = (a0 + a1) + (a2 + a3);
+  }
+  *reinterpret_cast<cs_f32x4*>(&part[ty][4 * tx]) = s;
+  __syncthreads();
+  const int64_t o = blk * CSQ_COLS + threadIdx.x;
+  if (threadIdx.x < CSQ_COLS && o < cols) {
+    float t = part[0][threadIdx.x];
+#pragma unroll
+    for (int k = 1; k < CS_SLICES; ++k) t += part[k][threadIdx.x];
+    uint32_t at = (uint32_t)o;
+    if (pt > 0) {
+      const uint32_t per_t = (uint32_t)pco * (uint32_t)pc, tt = at / per_t;
+      at = (at - tt * per_t) * (uint32_t)pt + tt;
+    }
+    out[at] = t;
+  }
+}
+
 }  // namespace novaq
