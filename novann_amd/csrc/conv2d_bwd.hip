@@ -582,12 +582,13 @@ __global__ __launch_bounds__(DW_THREADS, 2) void dweight_kernel(
 // of the stage index).  Two register sets: stage t + 2's loads are issued as
 // soon as stage t's registers are in LDS, so they have two stages' products
 // to arrive.  Staging, one of two forms:
-//   - VEC (zero padding, W and OW multiples of 4, 16-byte aligned tensors):
-//     16-byte loads of 4 consecutive grad pixels (one Gs row run, an 8-byte
-//     LDS write) or 4 consecutive input columns (two 4-byte LDS writes; xo is
-//     pw rounded up to even), items spread over all lanes (GU grad and XJ
-//     input items per lane); the padding columns of Xs are zeroed once and
-//     never written;
+//   - VW = 4 or 2 (zero padding, W and OW multiples of VW, 16-byte aligned
+//     tensors): loads of VW consecutive grad pixels (one run of a Gs row, an
+//     LDS write of 2 VW bytes) or VW consecutive input columns (4-byte LDS
+//     writes; xo is pw rounded up to even), items spread over all lanes (GU
+//     grad and XJ input items per lane); the padding columns of Xs are zeroed
+//     once and never written (128 -> 128 channels, 64 maps of 14 x 14, VW = 2:
+//     20.0 us, by slots 24.1);
 //   - otherwise one 4-byte slot at a time: a band's R * OW grad values and a
 //     channel's rows_in * XW staged slots spread over the 64 lanes of a wave
 //     (2 and XJ slots per lane), wave w taking channels w, w + DR_WAVES, ...
@@ -596,7 +597,8 @@ __global__ __launch_bounds__(DW_THREADS, 2) void dweight_kernel(
 constexpr int DR_K = 128;          // pixels per stage
 constexpr int DR_WAVES = 12;       // waves per workgroup (at most 12 taps)
 constexpr int DR_GC = 6, DR_XC = 3;  // grad / input channels a wave stages (12 x 6 >= 64, 12 x 3 >= 32)
-constexpr int DR_GU = 3;           // VEC: grad quads per lane (64 channels x 32 quads <= 3 x 768)
+// grad runs of VW pixels per lane (64 channels x 128 / VW runs over 768 lanes)
+constexpr int dr_gu(int vw) { return vw == 2 ? 6 : 3; }
 constexpr uint32_t DR_OOB = 0x80000000u;  // byte offset past any buffer (reads 0)
 constexpr uint32_t DR_BUF3 = 0x00020000u;  // buffer resource word 3 (raw, 32-bit data)
 constexpr int DR_FAR = 1 << 30;    // a row index no band reaches (masked item)
@@ -609,30 +611,32 @@ struct RowsGeom {
 };
 
 // One stage's loads in registers.
-template <bool VEC, int XJ>
+template <int VW, int XJ>
 struct RowsRegs {
+  typedef float Run __attribute__((ext_vector_type(VW)));
+  Run g[dr_gu(VW)];
+  Run x[XJ];
+};
+template <int XJ>
+struct RowsRegs<0, XJ> {
   float g[2 * DR_GC];
   float x[DR_XC * XJ];
 };
-template <int XJ>
-struct RowsRegs<true, XJ> {
-  f32x4 g[DR_GU];
-  f32x4 x[XJ];
-};
 
 // MODE 0: grad_weight; 1: grad_weight and grad_bias; 2: grad_bias only (no x,
-// no products).  grad_bias, in a fixed order: VEC: each lane adds each of its
-// grad quads ((v0 + v1) + (v2 + v3)) per stage in stage order, then the
-// quads of a channel are added in band order through LDS; otherwise each
+// no products).  grad_bias, in a fixed order: VW > 0: each lane adds each of its
+// grad runs (v0 + v1, or (v0 + v1) + (v2 + v3)) per stage in stage order, then
+// the runs of a channel are added in band order through LDS; otherwise each
 // lane adds the grad values it loads per channel in stage order and the wave
 // adds its 64 lanes in a fixed butterfly.  c block 0 writes the chunk's
 // per-channel sum to bpart.
-template <int XJ, int MODE, bool VEC>
+template <int XJ, int MODE, int VW>
 __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
     const float* __restrict__ grad, const float* __restrict__ x, float* __restrict__ part,
     float* __restrict__ bpart, BwdGeom g, RowsGeom rg, int chunks, int co_blocks,
     int c_blocks) {
-  constexpr bool WGT = MODE != 2, BIAS = MODE != 0;
+  constexpr bool WGT = MODE != 2, BIAS = MODE != 0, VEC = VW != 0;
+  constexpr int GU = dr_gu(VW), RUN = VEC ? VW : 1;
   constexpr int NT = DR_WAVES * 64;
   extern __shared__ __attribute__((aligned(16))) uint8_t dr_lds[];
   constexpr int GP = DR_K + 8;  // Gs row pitch (bf16); slot DR_K takes masked lanes
@@ -653,8 +657,8 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
   const int HW = g.H * g.W;
   const int P = g.OH * g.OW;
   const int xslots = rg.rows_in * rg.XW;
-  const int q4 = rg.R * g.OW / 4;  // VEC: grad quads of a band per channel
-  const int W4 = g.W / 4;
+  const int q4 = rg.R * g.OW / RUN;  // VEC: grad runs of a band per channel
+  const int W4 = g.W / RUN;
 
   f32x16 acc[2];
 #pragma unroll
@@ -669,17 +673,17 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
     const int words = VEC ? (64 * GP + 32 * rg.cp) / 2 : 64 * GP / 2;
     for (int i = tid; i < words; i += NT) z[i] = 0u;
   }
-  float bsum[VEC ? DR_GU : DR_GC];
+  float bsum[VEC ? GU : DR_GC];
 #pragma unroll
-  for (int i = 0; i < (VEC ? DR_GU : DR_GC); ++i) bsum[i] = 0.0f;
+  for (int i = 0; i < (VEC ? GU : DR_GC); ++i) bsum[i] = 0.0f;
 
-  // VEC items of this lane: grad quad u = channel co_l = it / q4, pixels
-  // 4 (it % q4) .. + 3 of the band (byte offset gbase before the band's,
-  // band row grow, Gs element gdst; DR_FAR / -1 when masked); input quad u =
-  // channel it / (rows_in W4), staged row xrr, input columns 4q .. 4q + 3
+  // VEC items of this lane: grad run u = channel co_l = it / q4, pixels
+  // VW (it % q4) .. of the band (byte offset gbase before the band's,
+  // band row grow, Gs element gdst; DR_FAR / -1 when masked); input run u =
+  // channel it / (rows_in W4), staged row xrr, input columns VW q ..
   // (byte offset xcb before the row's, Xs element xdst)
-  uint32_t gbase[DR_GU], xcb[XJ];
-  int grow[DR_GU], gdst[DR_GU], xrr[XJ], xdst[XJ];
+  uint32_t gbase[GU], xcb[XJ];
+  int grow[GU], gdst[GU], xrr[XJ], xdst[XJ];
   // scalar slots of this lane: Gs slot j = grad value m = lane + 64 j of the
   // band (row gr, Gs column gk: DR_K past the band); Xs slot j = staged row
   // xr, input column xw (-1: zero, also for columns no output of the band
@@ -690,9 +694,9 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
   uint32_t gch[DR_GC], xch[DR_XC];
   if constexpr (VEC) {
 #pragma unroll
-    for (int u = 0; u < DR_GU; ++u) {
+    for (int u = 0; u < GU; ++u) {
       const int it = tid + NT * u;
-      const int co_l = it / q4, m = 4 * (it - co_l * q4);
+      const int co_l = it / q4, m = RUN * (it - co_l * q4);
       const int r = m / g.OW, col = m - r * g.OW;
       const bool live = co_l < 64 && co0 + co_l < g.C_out;
       gbase[u] = (uint32_t)((co0 + co_l) * P + m) * 4u;
@@ -706,9 +710,9 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
       const int c_l = it / per, rest = it - c_l * per;
       const int rr = rest / W4, q = rest - rr * W4;
       const bool live = c_l < 32 && c0 + c_l < g.C;
-      xcb[u] = (uint32_t)((c0 + c_l) * HW + 4 * q) * 4u;
+      xcb[u] = (uint32_t)((c0 + c_l) * HW + RUN * q) * 4u;
       xrr[u] = live ? rr : DR_FAR;
-      xdst[u] = c_l < 32 ? c_l * rg.cp + rr * rg.XW + 4 * q + rg.xo : -1;
+      xdst[u] = c_l < 32 ? c_l * rg.cp + rr * rg.XW + RUN * q + rg.xo : -1;
     }
   } else {
 #pragma unroll
@@ -738,7 +742,12 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
     }
   }
 
-  typedef RowsRegs<VEC, XJ> Regs;
+  typedef RowsRegs<VW, XJ> Regs;
+  auto load_run = [](const __amdgpu_buffer_rsrc_t& buf, uint32_t off) {
+    if constexpr (VW == 2)
+      return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(buf, off, 0, 0));
+    else return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, off, 0, 0));
+  };
   // The loads of the stage of band s of image n, all in flight together.
   auto load_stage = [&](Regs& rv, int n, int s) {
     const int oh0 = s * rg.R;
@@ -751,9 +760,9 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
     if constexpr (VEC) {
       const uint32_t band = (uint32_t)(oh0 * g.OW) * 4u;
 #pragma unroll
-      for (int u = 0; u < DR_GU; ++u) {
+      for (int u = 0; u < GU; ++u) {
         const uint32_t off = grow[u] < rows_left ? gbase[u] + band : DR_OOB;
-        rv.g[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(gbuf, off, 0, 0));
+        rv.g[u] = load_run(gbuf, off);
       }
       if constexpr (WGT) {
 #pragma unroll
@@ -761,7 +770,7 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
           const int hi = oh0 - g.ph + xrr[u];
           const uint32_t off = (xrr[u] < rows_read && hi >= 0 && hi < g.H)
                                    ? xcb[u] + (uint32_t)(hi * g.W) * 4u : DR_OOB;
-          rv.x[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, off, 0, 0));
+          rv.x[u] = load_run(xbuf, off);
         }
       }
     } else {
@@ -793,7 +802,10 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
   auto add_bias = [&](const Regs& rv) {
     if constexpr (VEC) {
 #pragma unroll
-      for (int u = 0; u < DR_GU; ++u) bsum[u] += (rv.g[u][0] + rv.g[u][1]) + (rv.g[u][2] + rv.g[u][3]);
+      for (int u = 0; u < GU; ++u) {
+        if constexpr (VW == 2) bsum[u] += rv.g[u][0] + rv.g[u][1];
+        else bsum[u] += (rv.g[u][0] + rv.g[u][1]) + (rv.g[u][2] + rv.g[u][3]);
+      }
     } else {
 #pragma unroll
       for (int k = 0; k < 2 * DR_GC; ++k) bsum[k >> 1] += rv.g[k];
@@ -824,20 +836,28 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
     if constexpr (BIAS) add_bias(rv);
     if constexpr (VEC) {
 #pragma unroll
-      for (int u = 0; u < DR_GU; ++u) {
+      for (int u = 0; u < GU; ++u) {
         if (gdst[u] < 0) continue;
-        const f32x2 lo = {rv.g[u][0], rv.g[u][1]}, hi = {rv.g[u][2], rv.g[u][3]};
-        *reinterpret_cast<u32x2b*>(Gs + gdst[u]) =
-            u32x2b{__builtin_bit_cast(uint32_t, __builtin_convertvector(lo, bf16x2)),
-                   __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf16x2))};
+        const f32x2 lo = {rv.g[u][0], rv.g[u][1]};
+        const uint32_t l = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, bf16x2));
+        if constexpr (VW == 2) {
+          *reinterpret_cast<uint32_t*>(Gs + gdst[u]) = l;
+        } else {
+          const f32x2 hi = {rv.g[u][2], rv.g[u][3]};
+          *reinterpret_cast<u32x2b*>(Gs + gdst[u]) =
+              u32x2b{l, __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf16x2))};
+        }
       }
 #pragma unroll
       for (int u = 0; u < XJ; ++u) {
         if (xdst[u] < 0) continue;
-        const f32x2 lo = {rv.x[u][0], rv.x[u][1]}, hi = {rv.x[u][2], rv.x[u][3]};
+        const f32x2 lo = {rv.x[u][0], rv.x[u][1]};
         uint32_t* d = reinterpret_cast<uint32_t*>(Xs + xdst[u]);
         d[0] = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, bf16x2));
-        d[1] = __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf16x2));
+        if constexpr (VW == 4) {
+          const f32x2 hi = {rv.x[u][2], rv.x[u][3]};
+          d[1] = __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf16x2));
+        }
       }
     } else {
 #pragma unroll
@@ -887,11 +907,11 @@ __global__ __launch_bounds__(DR_WAVES * 64) void dweight_rows_kernel(
     }
   }
   if constexpr (BIAS && VEC) {
-    // the quads of each channel added in band order
+    // the runs of each channel added in band order
     float* red = reinterpret_cast<float*>(dr_lds);
     __syncthreads();  // the last stage's fragment reads are done
 #pragma unroll
-    for (int u = 0; u < DR_GU; ++u) {
+    for (int u = 0; u < GU; ++u) {
       const int it = tid + NT * u;
       if (it < 64 * q4) red[it] = bsum[u];
     }
@@ -1141,9 +1161,9 @@ size_t c1_geometry(const BwdGeom& g, D1Geom& d) {
 
 
 // The stride-1 rows path applies (its LDS bytes, input items or slots per
-// lane XJ, and whether its staging is VEC), or 0.  aligned: grad and x start
+// lane XJ, and the VW of its staging), or 0.  aligned: grad and x start
 // on 16 bytes (always through the C ABI, which requires it).
-size_t rows_geometry(const BwdGeom& g, bool aligned, RowsGeom& rg, int& xj, bool& vec) {
+size_t rows_geometry(const BwdGeom& g, bool aligned, RowsGeom& rg, int& xj, int& vw) {
   const int taps = g.KH * g.KW;
   // (fewer than 16 input channels leave most of the 32-channel tile idle: a
   // 1-channel 28x28 batch of 256 takes ~33 us here against 16.5 on dweight_kernel)
@@ -1161,14 +1181,19 @@ size_t rows_geometry(const BwdGeom& g, bool aligned, RowsGeom& rg, int& xj, bool
   const int xslots = rg.rows_in * rg.XW;
   rg.cp = xslots + 2;  // odd dword pitch; slot xslots is the spare
   rg.spi = (g.OH + rg.R - 1) / rg.R;
-  // VEC: input quads per lane; xo even (4-byte LDS writes), so xo + W and
+  // VW > 0: input runs per lane; xo even (4-byte LDS writes), so xo + W and
   // the columns the products read stay within XW (stride 1, KW <= 8)
-  const int vitems = 32 * rg.rows_in * (g.W / 4);
-  const int vj = std::max(2, (vitems + DR_WAVES * 64 - 1) / (DR_WAVES * 64));
-  vec = aligned && g.pad_mode == NOVAQ_PAD_ZEROS && g.W % 4 == 0 && g.OW % 4 == 0 &&
-        vj <= DR_MAX_XJ;
-  rg.xo = vec ? (g.pw + 1) & ~1 : g.pw;
-  xj = vec ? vj : (xslots + 63) / 64;
+  vw = 0;
+  int vj = 0;
+  for (int v = 4; v >= 2 && !vw; v -= 2) {
+    const int vitems = 32 * rg.rows_in * (g.W / v);
+    vj = std::max(2, (vitems + DR_WAVES * 64 - 1) / (DR_WAVES * 64));
+    if (aligned && g.pad_mode == NOVAQ_PAD_ZEROS && g.W % v == 0 && g.OW % v == 0 &&
+        vj <= DR_MAX_XJ)
+      vw = v;
+  }
+  rg.xo = vw ? (g.pw + 1) & ~1 : g.pw;
+  xj = vw ? vj : (xslots + 63) / 64;
   if (xj < 2 || xj > DR_MAX_XJ) return 0;  // (more slots per lane spill registers)
   const size_t bytes = (size_t)64 * (DR_K + 8) * 2 + (size_t)32 * rg.cp * 2;
   return bytes <= 150 * 1024 ? bytes : 0;
@@ -1352,9 +1377,9 @@ static int dweight_launch(const float* grad, const float* x, const BwdGeom& g, i
   // chunks, so its bits match a full call's)
   RowsGeom rg{};
   int xj = 0;
-  bool vec = false;
+  int vw = 0;
   const bool aligned = ((reinterpret_cast<uintptr_t>(grad) | reinterpret_cast<uintptr_t>(x)) & 15) == 0;
-  const size_t rows_lds = rows_geometry(g, aligned, rg, xj, vec);
+  const size_t rows_lds = rows_geometry(g, aligned, rg, xj, vw);
   if (rows_lds) {
     float* part = reinterpret_cast<float*>(base + ws.part);
     float* bpart = reinterpret_cast<float*>(base + ws.bpart);
@@ -1368,36 +1393,31 @@ static int dweight_launch(const float* grad, const float* x, const BwdGeom& g, i
     if (blocks > 0x7FFFFFFF) return NOVAQ_EINVAL;
     using RowsKernel = void (*)(const float*, const float*, float*, float*, BwdGeom, RowsGeom,
                                 int, int, int);
-    static const RowsKernel kerns[2][2][DR_MAX_XJ + 1] = {
-        {{nullptr, nullptr, dweight_rows_kernel<2, 0, false>, dweight_rows_kernel<3, 0, false>,
-          dweight_rows_kernel<4, 0, false>, dweight_rows_kernel<5, 0, false>},
-         {nullptr, nullptr, dweight_rows_kernel<2, 1, false>, dweight_rows_kernel<3, 1, false>,
-          dweight_rows_kernel<4, 1, false>, dweight_rows_kernel<5, 1, false>}},
-        {{nullptr, nullptr, dweight_rows_kernel<2, 0, true>, dweight_rows_kernel<3, 0, true>,
-          dweight_rows_kernel<4, 0, true>, dweight_rows_kernel<5, 0, true>},
-         {nullptr, nullptr, dweight_rows_kernel<2, 1, true>, dweight_rows_kernel<3, 1, true>,
-          dweight_rows_kernel<4, 1, true>, dweight_rows_kernel<5, 1, true>}}};
-    static bool lds_raised[2][2][DR_MAX_XJ + 1] = {};
+#define NOVAQ_ROWS_KERNELS(MODE, VW)                                        \
+  {nullptr, nullptr, dweight_rows_kernel<2, MODE, VW>, dweight_rows_kernel<3, MODE, VW>, \
+   dweight_rows_kernel<4, MODE, VW>, dweight_rows_kernel<5, MODE, VW>}
+    static const RowsKernel kerns[3][2][DR_MAX_XJ + 1] = {  // VW / 2
+        {NOVAQ_ROWS_KERNELS(0, 0), NOVAQ_ROWS_KERNELS(1, 0)},
+        {NOVAQ_ROWS_KERNELS(0, 2), NOVAQ_ROWS_KERNELS(1, 2)},
+        {NOVAQ_ROWS_KERNELS(0, 4), NOVAQ_ROWS_KERNELS(1, 4)}};
+#undef NOVAQ_ROWS_KERNELS
+    static bool lds_raised[3][2][DR_MAX_XJ + 1] = {};
     if (mode == 2) {
-      // the same grad reads and sums as a full call (VEC: the quads' sums
+      // the same grad reads and sums as a full call (VW > 0: the runs' sums
       // meet in LDS)
-      const size_t red = vec ? (size_t)64 * (rg.R * g.OW / 4) * 4 : 0;
-      if (vec)
-        hipLaunchKernelGGL((dweight_rows_kernel<2, 2, true>), dim3((unsigned)blocks),
-                           dim3(DR_WAVES * 64), red, stream, grad, x, part, bpart, g, rg,
-                           (int)rchunks, (int)co_blocks, 1);
-      else
-        hipLaunchKernelGGL((dweight_rows_kernel<2, 2, false>), dim3((unsigned)blocks),
-                           dim3(DR_WAVES * 64), 0, stream, grad, x, part, bpart, g, rg,
-                           (int)rchunks, (int)co_blocks, 1);
+      static const RowsKernel bias_kerns[3] = {dweight_rows_kernel<2, 2, 0>, dweight_rows_kernel<2, 2, 2>,
+                                               dweight_rows_kernel<2, 2, 4>};
+      const size_t red = vw ? (size_t)64 * (rg.R * g.OW / vw) * 4 : 0;
+      hipLaunchKernelGGL(bias_kerns[vw / 2], dim3((unsigned)blocks), dim3(DR_WAVES * 64), red,
+                         stream, grad, x, part, bpart, g, rg, (int)rchunks, (int)co_blocks, 1);
     } else {
-      const RowsKernel kern = kerns[vec][mode][xj];
-      if (!lds_raised[vec][mode][xj]) {
+      const RowsKernel kern = kerns[vw / 2][mode][xj];
+      if (!lds_raised[vw / 2][mode][xj]) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
                                                  150 * 1024);
         if (e != hipSuccess) return hip_fail(e);
-        lds_raised[vec][mode][xj] = true;
+        lds_raised[vw / 2][mode][xj] = true;
       }
       hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(DR_WAVES * 64), rows_lds, stream, grad,
                          x, part, bpart, g, rg, (int)rchunks, (int)co_blocks, (int)c_blocks);
