@@ -26,14 +26,13 @@
 //     operand gathered element-wise with the padding mode resolved); each
 //     workgroup writes one partial grad_weight tile to the workspace, and the
 //     first j block also the per-channel grad sums of its chunk (grad_bias);
-//   - finish_kernel: one launch that adds the chunk partials in a fixed order
-//     (novaq_colsum.h's column sum, so results do not depend on scheduling;
-//     16 columns a workgroup with one input channel, else 64); with one input
-//     channel and grad_input on the one-output-channel kernel, c1_tail_kernel
-//     instead: the same sums beside grad_input's bands, the weight read
-//     flipped in place
-//     for grad_weight and grad_bias, and flips the weights for grad_input;
-//     grad_input's convolution runs after it.
+//   - finish_kernel: one launch that adds the chunk partials of grad_weight and
+//     grad_bias in a fixed order (novaq_colsum.h's column sum, so results do
+//     not depend on scheduling; 16 columns a workgroup with one input channel,
+//     256 where that many cover the CUs, else 64) and flips the weights for
+//     grad_input, whose convolution runs after it; with one input channel and
+//     grad_input on the one-output-channel kernel, c1_tail_kernel instead: the
+//     same sums beside grad_input's bands, the weight read flipped in place.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

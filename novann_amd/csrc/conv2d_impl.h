@@ -1402,7 +1402,7 @@ struct SmallGeom {
   int vec;      // OW % 4 == 0: whole chunks, vector stores
 };
 
-// F3: a 3 x 3 window with zeros padding (config [5]'s conv1), its loops and
+// F3: a 3 x 3 window with zeros padding, its loops and
 // padding tests fixed at compile time; other windows and modes take F3 = false.
 template <int WT, int XT, bool VEC, bool F3>
 __global__ __launch_bounds__(256) void conv2d_smallc_kernel(

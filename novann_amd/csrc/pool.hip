@@ -962,7 +962,7 @@ __global__ __launch_bounds__(256) void max_pool2d_bwd_tile_kernel(
 }
 
 // 2 x 2 windows, stride 2, no padding, H and W even (every input element in
-// exactly one window: config [5]'s MaxPool2d(2, 2)): lane t makes window t's
+// exactly one window): lane t makes window t's
 // four gradients, its two input rows read as 2-element loads and its two
 // gradient rows written as 8-byte stores (x aligned to 2 elements, gi to 8
 // bytes).  t < 2^31: the divisions by the plane's windows and by OW are
