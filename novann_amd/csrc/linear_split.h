@@ -50,6 +50,7 @@
 #include "novaq_convert.h"
 #include "novaq_epilogue.h"
 #include "novaq_internal.h"
+#include "novaq_split_index.h"
 #include "novaq_xload.h"
 
 namespace novaq {
@@ -209,6 +210,7 @@ struct LsRow {
   }
   // index of the operand's element that tile t, lane row r holds
   __device__ __forceinline__ int index(const int t, int r) const { return 16 * t + r; }
+  __device__ __forceinline__ bool owns(const int, int) const { return true; }
 };
 
 // Row operand of a small tile, read 64 contiguous bytes a quad of lanes: a
@@ -313,7 +315,7 @@ struct LsCol {
   __device__ __forceinline__ void init(const uint8_t* p, int64_t pitch_, int i0, int count, int lane) {
     kl = (lane >> 4) * 16;
     pitch = pitch_;
-    last = count - T - i0;
+    last = split_detail::col_last(T, count, i0);
     base = p + kl * pitch + (int64_t)(i0 + index(0, lane & 15)) * bits / 8;
   }
   __device__ __forceinline__ Run load_run(int64_t off) const {
@@ -367,10 +369,15 @@ struct LsCol {
       return ls_decode8<DT>(w);
     }
   }
-  // A run that would pass the last index starts T before it instead: those
-  // lanes repeat elements of the lanes before them (the same sums, stored
-  // twice), so edge tiles take the same vector loads.
-  __device__ __forceinline__ int index(const int t, int r) const { return min(T * r, last) + t; }
+  // A run that would pass the last index starts T before it instead, so edge
+  // tiles take the same vector loads; what such a run repeats, or holds of the
+  // tile before, is summed and not stored (owns).
+  __device__ __forceinline__ int index(const int t, int r) const {
+    return split_detail::col_index(T, last, t, r);
+  }
+  __device__ __forceinline__ bool owns(const int t, int r) const {
+    return split_detail::col_owns(T, last, t, r);
+  }
   // fp32 only: the sum of these 8 k of tile t's element, in K order
   static __device__ __forceinline__ float sum(const Regs& r, const int t) {
     static_assert(bits == 32, "fp32 operand");
@@ -573,7 +580,8 @@ __global__ __launch_bounds__(NWV * 64) void linear_split_kernel(
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) mine[wo.index(j, q4 + q)] = acc[i][j][q];
+        for (int j = 0; j < NT; ++j)
+          if (wo.owns(j, q4 + q)) mine[wo.index(j, q4 + q)] = acc[i][j][q];
     } else {
 #pragma unroll
       for (int j = 0; j < NT; ++j) *reinterpret_cast<ls_f32x4*>(mine + 16 * j + q4) = acc[i][j];
@@ -582,7 +590,7 @@ __global__ __launch_bounds__(NWV * 64) void linear_split_kernel(
     for (int o = tid; o < 16 * TN / 4; o += NWV * 64) {
       const int r = o / (TN / 4), c = (o - r * (TN / 4)) * 4;
       const int m = m0 + xo.index(i, r), n = n0 + c;
-      if (m >= g.M || n >= g.N) continue;
+      if (m >= g.M || n >= g.N || !xo.owns(i, r)) continue;
       ls_f32x4 v = *reinterpret_cast<const ls_f32x4*>(part + r * LP + c);
 #pragma unroll
       for (int k = 1; k < NWV; ++k)
@@ -616,7 +624,7 @@ __global__ __launch_bounds__(NWV * 64) void linear_split_kernel(
         float v = xs[i];
         v += __shfl_xor(v, 16);
         v += __shfl_xor(v, 32);
-        if (lane < 16) part[wave * 16 * MT + xo.index(i, lane)] = v;
+        if (lane < 16 && xo.owns(i, lane)) part[wave * 16 * MT + xo.index(i, lane)] = v;
       }
       __syncthreads();
       for (int o = tid; o < 16 * MT; o += NWV * 64) {

@@ -75,6 +75,18 @@ def test_backward_exact_operands(n, d_in, d_out, wdt):
     check(gb.cpu().numpy().reshape(1, -1), np.ones((1, n)), g.astype(np.float64), "grad_bias")
 
 
+# One to T - 1 indices of W's columns (D_in), of x's and of grad's left for the
+# last tile of T-wide runs: T = 2 (32 x 32 tiles), 4 (64 x 64) and both (64 x 32).
+EDGES = [(5, 33, 97), (40, 65, 33), (1024, 1025, 44), (1023, 1026, 36), (1025, 1027, 20),
+         (20, 1024, 1025), (12, 1025, 1026), (9, 1057, 1027)]
+
+
+@pytest.mark.parametrize("wdt", ["e4m3", "e2m1", "f32"])
+@pytest.mark.parametrize("n,d_in,d_out", EDGES)
+def test_backward_of_a_few_indices_past_a_tile(n, d_in, d_out, wdt):
+    test_backward_exact_operands(n, d_in, d_out, wdt)
+
+
 # more than 32 tiles of 128 x 256, ragged in M, N and K
 RAGGED = [(1026, 144, 1003), (1100, 32, 1280), (1024, 416, 1025), (4100, 160, 250)]
 
