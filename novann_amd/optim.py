@@ -100,6 +100,11 @@ class AdamW:
             is_bn_param = getattr(p, "name", None) in ("gamma", "beta")
             hp = _lib.AdamW(self.lr, self.b1, self.b2, self.eps, self.wd, self.t,
                             0 if is_bn_param else 1)
+            # (the raw lookup below takes a host tensor's device as "the current
+            # one"; the kernels would then follow host pointers)
+            if not w.is_cuda:
+                raise ValueError(f"AdamW: parameters must be CUDA (HIP) device tensors, got one "
+                                 f"on {w.device}")
             stream = torch._C._cuda_getCurrentRawStream(w.get_device())
             if w.dtype == torch.float64:
                 g, g32 = _dev_grad64(p.grad, w.device)

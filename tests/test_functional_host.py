@@ -78,3 +78,29 @@ def test_storage_size_checks():
         quant._require_holds(torch.empty(2, dtype=torch.uint8), "e2m1", 5, "x")
     with pytest.raises(ValueError, match="need"):
         quant._require_holds(torch.empty(7, dtype=torch.int16), "f16", 8, "x")
+
+
+def test_adamw_refuses_host_tensors(monkeypatch):
+    """A host tensor as a parameter or a master raises ValueError at the step:
+    no kernel is given its address."""
+    import torch
+
+    from novann_amd import optim
+    from novann_amd.module import QuantizedParameters
+
+    class NoCalls:
+        def __getattr__(self, name):
+            raise AssertionError(f"{name} called with host memory")
+
+    monkeypatch.setattr(optim, "_device", lambda: torch.device("cpu"))
+    monkeypatch.setattr(optim._lib, "load", NoCalls)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0)
+    p = Parameters(np.zeros(1, np.float32))
+    p.data = torch.zeros(4, 8)
+    q = QuantizedParameters(torch.zeros(32, dtype=torch.uint8), (4, 8), "e4m3", torch.ones(1),
+                            master=torch.zeros(4, 8))
+    for param in (p, q):
+        opt = optim.AdamW([param], lr=1e-3)
+        param.grad = torch.zeros(4, 8)
+        with pytest.raises(ValueError, match="device tensors"):
+            opt.step()
