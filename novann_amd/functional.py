@@ -168,7 +168,7 @@ def _epilogue_args(ep: Optional[Epilogue], channels: int, dev: torch.device):
             torch.cuda.is_current_stream_capturing():
         t = _upload_rows(host, channels, dev)
         keep.append(t)
-        rows = iter(range(t.data_ptr(), t.data_ptr() + 4 * t.numel(), 4 * t.shape[1]))
+        rows = iter([t.data_ptr() + 4 * t.shape[1] * i for i in range(len(host))])
 
     def chan(a, what):
         if a is None:

@@ -104,3 +104,26 @@ def test_adamw_refuses_host_tensors(monkeypatch):
         param.grad = torch.zeros(4, 8)
         with pytest.raises(ValueError, match="device tensors"):
             opt.step()
+
+
+@pytest.mark.parametrize("channels", [0, 1, 5, 8])
+def test_epilogue_vectors_of_any_channel_count(monkeypatch, channels):
+    """Host-array channel vectors lie in one upload, each on a 16-byte
+    boundary; no channels (a layer without outputs) is a count like others."""
+    import torch
+
+    sent = []
+
+    def upload(arrays, n, dev):
+        sent.append(torch.zeros((len(arrays), (n + 3) // 4 * 4)))
+        return sent[-1]
+
+    monkeypatch.setattr(F, "_upload_rows", upload)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    ep = F.Epilogue(channel_mul=np.ones(channels, np.float32),
+                    channel_add=np.ones(channels, np.float32))
+    st, _, keep = F._epilogue_args(ep, channels, torch.device("cpu"))
+    assert len(sent) == 1 and keep[0] is sent[0]
+    if channels:
+        assert st.channel_mul == sent[0][0].data_ptr()
+        assert st.channel_add == sent[0][1].data_ptr()

@@ -52,3 +52,12 @@ def test_device_and_host_vectors_mix_and_sizes_are_checked():
             F.linear(x, q, epilogue=F.Epilogue(**bad))
     with pytest.raises(TypeError):
         F.linear(x, q, epilogue=F.Epilogue(channel_mul=[1.0] * 6))
+
+
+def test_layer_without_outputs_takes_empty_vectors():
+    x = torch.zeros((3, 8), device="cuda")
+    w = torch.zeros((0, 8), device="cuda")
+    none = np.zeros(0, np.float32)
+    for kw in (dict(channel_mul=none), dict(channel_add=none),
+               dict(channel_mul=none, channel_add=none, relu=True)):
+        assert F.linear(x, w, epilogue=F.Epilogue(**kw)).shape == (3, 0)
