@@ -1400,7 +1400,7 @@ static int dweight_launch(const float* grad, const float* x, const BwdGeom& g, i
         {NOVAQ_ROWS_KERNELS(0, 2), NOVAQ_ROWS_KERNELS(1, 2)},
         {NOVAQ_ROWS_KERNELS(0, 4), NOVAQ_ROWS_KERNELS(1, 4)}};
 #undef NOVAQ_ROWS_KERNELS
-    static bool lds_raised[3][2][DR_MAX_XJ + 1] = {};
+    static DeviceFlags raised[3][2][DR_MAX_XJ + 1];
     if (mode == 2) {
       // the same grad reads and sums as a full call (VW > 0: the runs' sums
       // meet in LDS)
@@ -1411,13 +1411,9 @@ static int dweight_launch(const float* grad, const float* x, const BwdGeom& g, i
                          stream, grad, x, part, bpart, g, rg, (int)rchunks, (int)co_blocks, 1);
     } else {
       const RowsKernel kern = kerns[vw / 2][mode][xj];
-      if (!lds_raised[vw / 2][mode][xj]) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 150 * 1024);
-        if (e != hipSuccess) return hip_fail(e);
-        lds_raised[vw / 2][mode][xj] = true;
-      }
+      const int rc = allow_lds(raised[vw / 2][mode][xj], reinterpret_cast<const void*>(kern),
+                               rows_lds, 150 * 1024);
+      if (rc != NOVAQ_OK) return rc;
       hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(DR_WAVES * 64), rows_lds, stream, grad,
                          x, part, bpart, g, rg, (int)rchunks, (int)co_blocks, (int)c_blocks);
     }

@@ -425,13 +425,9 @@ int chunk_launch_tile(const uint8_t* x, const float* x_scale, const uint8_t* w,
                       const float* w_scale, const Epilogue& ep, void* y, const ChunkGeom& g,
                       size_t lds, hipStream_t stream) {
   auto kern = conv2d_chunk_kernel<WT, XT, T, NCO, WCO, IPT>;
-  static bool raised = false;  // per instantiation
-  if (!raised && lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
-    if (e != hipSuccess) return hip_fail(e);
-    raised = true;
-  }
+  static DeviceFlags raised;  // per instantiation
+  const int rc = allow_lds(raised, reinterpret_cast<const void*>(kern), lds, 80 * 1024);
+  if (rc != NOVAQ_OK) return rc;
   hipLaunchKernelGGL(kern, dim3((unsigned)(g.groups * g.bands * g.tiles_m)), dim3(256), lds, stream,
                      x, x_scale, w, w_scale, ep, y, g);
   return check_launch();

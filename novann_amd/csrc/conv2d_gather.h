@@ -305,14 +305,10 @@ int gather_launch_tile(const uint8_t* x, const float* x_scale, const uint8_t* w,
   const size_t lds = table > out ? table : out;
   constexpr size_t MOST = 16 * MT * (4 * TN + 4) * 4 > CG_MAX_K * 4 ? 16 * MT * (4 * TN + 4) * 4
                                                                     : CG_MAX_K * 4;
-  static bool raised = MOST <= 64 * 1024;  // per instantiation: raise the limit once
+  static DeviceFlags raised;  // per instantiation
   auto kern = conv2d_gather_kernel<WT, XT, MT, NT>;
-  if (!raised) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)MOST);
-    if (e != hipSuccess) return hip_fail(e);
-    raised = true;
-  }
+  const int rc = allow_lds(raised, reinterpret_cast<const void*>(kern), lds, MOST);
+  if (rc != NOVAQ_OK) return rc;
   hipLaunchKernelGGL(kern, dim3((unsigned)(tm * tn)), dim3(256), lds, stream, x, x_scale, w,
                      w_scale, ep, y, g);
   return check_launch();

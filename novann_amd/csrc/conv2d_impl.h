@@ -1112,13 +1112,9 @@ int launch_band(const uint8_t* x, const float* x_scale, const void* w, const flo
                 const Epilogue& ep, void* y, const BandGeom& b, size_t lds, int64_t co_blocks,
                 hipStream_t stream) {
   auto kern = conv2d_band_kernel<WT, XT, IPT, K9>;
-  static size_t lds_enabled = 64 * 1024;  // per instantiation: raise the limit once
-  if (lds > lds_enabled) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_LIMIT);
-    if (e != hipSuccess) return hip_fail(e);
-    lds_enabled = LDS_LIMIT;
-  }
+  static DeviceFlags raised;  // per instantiation
+  const int rc = allow_lds(raised, reinterpret_cast<const void*>(kern), lds, LDS_LIMIT);
+  if (rc != NOVAQ_OK) return rc;
   const int64_t blocks = (int64_t)b.N * b.bands;
   if (blocks > 0x7FFFFFFF) return NOVAQ_EINVAL;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)co_blocks), dim3(THREADS), lds, stream,
@@ -1760,13 +1756,9 @@ int launch(const uint8_t* x, const float* x_scale, const void* w, const float* w
     return check_launch();
   }
   auto kern = conv2d_kernel<WT, XT>;
-  static size_t lds_enabled = 64 * 1024;  // per instantiation: raise the limit once
-  if (lds > lds_enabled) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_LIMIT);
-    if (e != hipSuccess) return hip_fail(e);
-    lds_enabled = LDS_LIMIT;
-  }
+  static DeviceFlags raised;  // per instantiation
+  const int rc = allow_lds(raised, reinterpret_cast<const void*>(kern), lds, LDS_LIMIT);
+  if (rc != NOVAQ_OK) return rc;
   int64_t grid = (int64_t)device_cu_count() * CONV_OCC;
   if (grid > g.tiles) grid = g.tiles;
   if (grid < 1) grid = 1;

@@ -1131,14 +1131,10 @@ template <int WT, int XT>
 int launch_f8(const uint8_t* x, const float* x_scale, int64_t M, int64_t K, const uint8_t* w,
               const float* w_scale, const Epilogue& ep, int64_t N, void* y, hipStream_t stream) {
   using D = F8<WT, XT>;
-  static bool lds_raised = false;
-  if (!lds_raised) {
-    const hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&linear_f8_kernel<WT, XT>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, D::lds);
-    if (e != hipSuccess) return hip_fail(e);
-    lds_raised = true;
-  }
+  static DeviceFlags raised;  // per instantiation
+  const int rc = allow_lds(raised, reinterpret_cast<const void*>(&linear_f8_kernel<WT, XT>), D::lds,
+                           D::lds);
+  if (rc != NOVAQ_OK) return rc;
   const int64_t tiles_m = M / BM, tiles_n = N / 256;
   hipLaunchKernelGGL((linear_f8_kernel<WT, XT>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512),
                      D::lds, stream, x, x_scale, w, w_scale, ep, y, (int)M, (int)N, (int)K,

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "../../include/novaq.h"
+#include "novaq_device_flags.h"
 
 namespace novaq {
 
@@ -57,6 +58,22 @@ int hip_fail(hipError_t e);
 inline int check_launch() {
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? NOVAQ_OK : hip_fail(e);
+}
+
+// Before a launch of kern with `lds` bytes of dynamic LDS: above the 64 KB that
+// every kernel may have, raises its limit to `limit` -- once on each device, the
+// limit being the device's, and with flags that several threads may reach at
+// once (`raised`: one object a kernel).
+inline int allow_lds(DeviceFlags& raised, const void* kern, size_t lds, size_t limit) {
+  if (lds <= 64 * 1024) return NOVAQ_OK;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return hip_fail(e);
+  if (raised.test(dev)) return NOVAQ_OK;
+  e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)limit);
+  if (e != hipSuccess) return hip_fail(e);
+  raised.set(dev);
+  return NOVAQ_OK;
 }
 
 // Compute units of the current device (cached per device).
