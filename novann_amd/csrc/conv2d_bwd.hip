@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) void dinput_phase_kernel(const float* __restri
   // pixels (h0 + sh i, w0 + sw j); taps a, a + sh, ... and b, b + sw, ...
   const int h0 = phase / min(g.sw, g.W), w0 = phase - h0 * min(g.sw, g.W);
   const int a = (h0 + g.ph) % g.sh, b = (w0 + g.pw) % g.sw;
-  const int Hp = (g.H - h0 + g.sh - 1) / g.sh, Wp = (g.W - w0 + g.sw - 1) / g.sw;
+  const int Hp = (g.H - 1 - h0) / g.sh + 1, Wp = (g.W - 1 - w0) / g.sw + 1;
   const int64_t total = (int64_t)g.N * Hp * Wp;
   const int64_t first = (int64_t)(rest - layer * blocks) * LANES;
   if (first >= total) return;  // the whole workgroup
@@ -239,10 +239,13 @@ __global__ __launch_bounds__(256) void dinput_phase_kernel(const float* __restri
     co0 += DI_CO;
     if (co0 >= g.C_out) {
       co0 = 0;
-      kw += g.sw;
-      if (kw >= g.KW) {
+      // (a stride is compared with the taps left before it is added: it may be
+      // as large as an int)
+      if (g.sw < g.KW - kw) {
+        kw += g.sw;
+      } else {
         kw = b;
-        kh += g.sh;
+        kh = g.sh < g.KH - kh ? kh + g.sh : g.KH;
       }
     }
     if (kh < g.KH) fetch(kh, kw, co0);

@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 import torch
 
+from novann_amd import _lib
 from novann_amd import functional as F
 from novann_amd.module import Parameters, QuantizedParameters
 from oracle import functional_ref as R
@@ -74,3 +75,34 @@ def test_nan_weight_reaches_only_its_taps_pixels():
     hit[:, 5, 1:7:2, 1:7:2] = True  # pixels 2 oh - 1 of tap (0, 0), oh = 1, 2, 3
     assert np.array_equal(np.isnan(got), hit)
     assert np.array_equal(got[~hit], clean[~hit])
+
+
+@pytest.mark.parametrize("stride", [(2**31 - 1, 2**31 - 1), (2**31 - 1, 2), (3, 2**31 - 3)])
+def test_strides_up_to_the_largest_int(stride):
+    """One output row (column): only the first window's pixels get a gradient,
+    every other pixel is zero, and no tap past the window is looked for."""
+    n, c, h, w, co, k, pad = 2, 17, 6, 9, 5, 3, (1, 1)
+    rng = np.random.default_rng(2)
+    wt = (rng.standard_normal((co, c, k, k)) * 0.1).astype(np.float32)
+    q = QuantizedParameters.from_float(wt, "e4m3")
+    oh, ow = ((d + 2 * p - k) // s + 1 for d, p, s in zip((h, w), pad, stride))
+    g = rng.standard_normal((n, co, oh, ow)).astype(np.float32)
+    gi = torch.full((n, c, h, w), float("nan"), device="cuda")
+    lib, gd = _lib.load(), torch.from_numpy(g).cuda()
+    code = _lib.DTYPES["e4m3"]
+    work = torch.empty(lib.novaq_conv2d_backward_workspace(n, c, co, k, k, code) + 16,
+                       dtype=torch.uint8, device="cuda")
+    # grad_input alone
+    _lib.check(lib.novaq_conv2d_backward(
+        gd.data_ptr(), None, n, c, h, w, q.codes.data_ptr(), code, q.scale.data_ptr(), co, k, k,
+        *stride, *pad, 0, gi.data_ptr(), None, None, work.data_ptr(), work.numel(),
+        torch.cuda.current_stream().cuda_stream), "conv2d backward")
+    # the same windows at a stride that fits the padded image
+    near = tuple(min(s, d + 2 * p) for s, d, p in zip(stride, (h, w), pad))
+    w64 = q.dequantize().cpu().numpy().astype(np.float64)
+    x64, g64 = np.zeros((n, c, h, w)), g.astype(np.float64)
+    want = R.conv2d_backward(g64, x64, w64, near, pad)[0]
+    size = R.conv2d_backward(np.abs(g64), x64, np.abs(w64), near, pad)[0]
+    got = gi.cpu().numpy()
+    assert np.all(np.abs(got - want) <= (co * k * k + 2) * 2.0**-24 * size + 1e-30)
+    assert not got[size == 0].any()
