@@ -24,9 +24,9 @@
 //     workgroup of 8 waves, K blocks of 128 (one 128-byte line of an FP8 W
 //     row), W raw in LDS and decoded per MFMA fragment, buffer loads with
 //     SGPR offsets;
-//   - linear_pipe_kernel (16-bit weights, or FP8 x and W, in whole 128-row
-//     tiles, K % 64): W decoded once per workgroup into bf16 LDS tiles, loads
-//     kept up to 3 K blocks ahead;
+//   - linear_pipe_kernel (M % 128, N % 128, K % 64, where the kernels above do
+//     not have whole tiles): W decoded once per workgroup into bf16 LDS tiles,
+//     loads kept up to 3 K blocks ahead;
 //   - linear_split_kernel (linear_split.h): any shape and format; small tiles
 //     with K split over the waves, for products of few rows or too few wide
 //     tiles to fill the chip, and for rows the others cannot read.
@@ -1168,6 +1168,28 @@ int launch(const uint8_t* x, const float* x_scale, int64_t M, int64_t K, const v
   }
   const dim3 grid((unsigned)(tiles_m * tiles_n));
   if (wide_preferred(M, N) && K > 0) {
+    // Whole tiles of 128 rows, 128 columns and 64 K that are not also whole
+    // tiles of the kernels below (and 16-bit weights, which those do not take):
+    // the staged-decode kernel; the ragged forms below pad K to 128 and the
+    // columns to 256 and store value by value.  fp32 x, E4M3 W: 4096 x 64 x 4096
+    // 19.5 us (ragged 33.3), 1024 x 1088 x 2304 19.6 (30.6), 65536 x 256 x 128
+    // 17.7 (44.0), 2048 x 4096 x 4224 124.6 (135.2); no shape measured the other
+    // way (K to 4160; FP4 W, bf16 and E4M3 x alike).
+    if constexpr (WT != F32) {
+      constexpr bool TILES = WT == E2M1 || (dtype_bits(WT) == 8 && XL<XT>::bytes >= 2);
+      if (rows_whole && N % 128 == 0 && K % BK == 0 && !(TILES && whole && K <= (1 << 21))) {
+        if (N % 256 == 0)
+          hipLaunchKernelGGL((linear_pipe_kernel<WT, XT, 256, 8, 1, 3>), grid, dim3(512), 0, stream,
+                             x, x_scale, wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
+                             (int)tiles_n);
+        else
+          hipLaunchKernelGGL((linear_pipe_kernel<WT, XT, 128, 4, 2, 2>),
+                             dim3((unsigned)(tiles_m * (N / 128))), dim3(256), 0, stream, x, x_scale,
+                             wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
+                             (int)(N / 128));
+        return check_launch();
+      }
+    }
     // W tile (256 rows of K codes) and x tile bytes must fit the buffer range;
     // ragged shapes need 16-byte chunks of W whole
     if constexpr ((WT == E4M3 || WT == E5M2) && XL<XT>::bytes >= 2) {
@@ -1193,21 +1215,6 @@ int launch(const uint8_t* x, const float* x_scale, int64_t M, int64_t K, const v
           hipLaunchKernelGGL((linear_wide_kernel<WT, XT, true>), grid, dim3(512), 0, stream, x,
                              x_scale, wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
                              (int)tiles_n);
-        return check_launch();
-      }
-    }
-    if constexpr (WT == BF16 || WT == F16 || (dtype_bits(WT) == 8 && XL<XT>::bytes == 1)) {
-      if (rows_whole && N % 256 == 0 && K % BK == 0) {
-        hipLaunchKernelGGL((linear_pipe_kernel<WT, XT, 256, 8, 1, 3>), grid, dim3(512), 0, stream,
-                           x, x_scale, wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
-                           (int)tiles_n);
-        return check_launch();
-      }
-      if (rows_whole && N % 128 == 0 && K % BK == 0) {
-        hipLaunchKernelGGL((linear_pipe_kernel<WT, XT, 128, 4, 2, 2>),
-                           dim3((unsigned)(tiles_m * (N / 128))), dim3(256), 0, stream, x, x_scale,
-                           wq, w_scale, ep, y, (int)M, (int)N, (int)K, (int)tiles_m,
-                           (int)(N / 128));
         return check_launch();
       }
     }

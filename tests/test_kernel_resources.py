@@ -50,3 +50,15 @@ def test_band_convolution_keeps_four_workgroups_per_cu(res):
     assert band
     for name, r in band.items():
         assert r["occupancy"] >= 4 and r.get("scratch", 0) == 0, (name, r)
+
+
+def test_staged_decode_products_cover_every_weight_format(res):
+    """Whole 128-row tiles that the wider tiles' kernels do not have run on the
+    staged-decode kernel at both of its tile widths, for every stored weight but
+    fp32 and every stored x."""
+    have = {n for n in res if "linear_pipe_kernel" in n}
+    for wt in (1, 2, 3, 4, 5):
+        for xt in range(5):
+            for bn in (256, 128):
+                assert any(f"linear_pipe_kernelILi{wt}ELi{xt}ELi{bn}E" in n for n in have), \
+                    (wt, xt, bn)
