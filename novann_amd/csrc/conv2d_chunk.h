@@ -31,6 +31,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "linear_split.h"
 #include "novaq_convert.h"
@@ -433,33 +434,45 @@ int chunk_launch_tile(const uint8_t* x, const float* x_scale, const uint8_t* w,
   return check_launch();
 }
 
-// The shape's bands and their launch for one tile, if it gives at least
-// `least` workgroups.
-template <int WT, int XT, int T, int NCO, int WCO>
-bool chunk_try(const uint8_t* x, const float* x_scale, const uint8_t* w, const float* w_scale,
-               const Epilogue& ep, void* y, ChunkGeom g, int least, hipStream_t stream, int* rc) {
-  int ipt = 0;
-  size_t lds = 0;
-  if (!chunk_geometry<WT, T>(g, 64 * (4 / WCO), 16 * NCO * WCO, &ipt, &lds)) return false;
-  if ((int64_t)g.groups * g.bands * g.tiles_m < least) return false;
-  *rc = ipt <= 1 ? chunk_launch_tile<WT, XT, T, NCO, WCO, 1>(x, x_scale, w, w_scale, ep, y, g, lds, stream)
-                 : chunk_launch_tile<WT, XT, T, NCO, WCO, 2>(x, x_scale, w, w_scale, ep, y, g, lds, stream);
-  return true;
-}
+// A shape's bands and images on one of the kernel's tiles: 0 = 32 channels x 256
+// pixels, 1 = 128 x 128, 2 = 64 x 128 a workgroup.
+struct ChunkPlan {
+  ChunkGeom g;
+  int tile, ipt;
+  size_t lds;
+  int64_t blocks() const { return (int64_t)g.groups * g.bands * g.tiles_m; }
+};
 
 // 64 channels x 128 pixels a workgroup; 32 x 256 for at most 32 channels; 128 x
 // 128 for a strided window over many channels, whose staged region is several
-// times its pixels and would be staged once per 64 channels.
+// times its pixels and would be staged once per 64 channels, where that gives
+// `wide_least` workgroups.
+template <int WT, int T>
+bool chunk_plan(const ChunkGeom& g, int wide_least, ChunkPlan& p) {
+  auto tile = [&](int id, int nco, int wco) {
+    p.g = g;
+    p.tile = id;
+    return chunk_geometry<WT, T>(p.g, 64 * (4 / wco), 16 * nco * wco, &p.ipt, &p.lds);
+  };
+  if (g.M <= 32) return tile(0, 2, 1);
+  if (T == 9 && g.M > 64 && g.sh * g.sw > 1 && tile(1, 4, 2) && p.blocks() >= wide_least) return true;
+  return tile(2, 2, 2);
+}
+
 template <int WT, int XT, int T>
-bool chunk_launch(const uint8_t* x, const float* x_scale, const uint8_t* w, const float* w_scale,
-                  const Epilogue& ep, void* y, const ChunkGeom& g, int least, hipStream_t stream,
-                  int* rc) {
-  if (g.M <= 32)
-    return chunk_try<WT, XT, T, 2, 1>(x, x_scale, w, w_scale, ep, y, g, least, stream, rc);
-  if (T == 9 && g.M > 64 && g.sh * g.sw > 1 &&
-      chunk_try<WT, XT, T, 4, 2>(x, x_scale, w, w_scale, ep, y, g, 4 * least, stream, rc))
-    return true;
-  return chunk_try<WT, XT, T, 2, 2>(x, x_scale, w, w_scale, ep, y, g, least, stream, rc);
+int chunk_launch(const uint8_t* x, const float* x_scale, const uint8_t* w, const float* w_scale,
+                 const Epilogue& ep, void* y, const ChunkPlan& p, hipStream_t stream) {
+  auto go = [&](auto nco, auto wco) {
+    constexpr int N = decltype(nco)::value, C = decltype(wco)::value;
+    return p.ipt <= 1
+               ? chunk_launch_tile<WT, XT, T, N, C, 1>(x, x_scale, w, w_scale, ep, y, p.g, p.lds, stream)
+               : chunk_launch_tile<WT, XT, T, N, C, 2>(x, x_scale, w, w_scale, ep, y, p.g, p.lds, stream);
+  };
+  if (p.tile == 0) return go(std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
+  if constexpr (T == 9) {
+    if (p.tile == 1) return go(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
+  }
+  return go(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
 }
 
 }  // namespace

@@ -1630,21 +1630,75 @@ bool launch_smallc(const uint8_t* x, const float* x_scale, const void* w, const 
   return true;
 }
 
-// The chunked path where it takes the shape with at least `least` workgroups;
-// returns false otherwise.
-template <int WT, int XT>
-bool launch_chunk(const uint8_t* x, const float* x_scale, const void* w, const float* w_scale,
-                  const Epilogue& ep, void* y, const ConvGeom& cg, int least, hipStream_t stream,
-                  int* rc) {
+// The chunked path's plan for the shape, or false where it does not take it.
+template <int WT>
+bool plan_chunk(const ConvGeom& cg, ChunkPlan& p) {
   if ((cg.pad_mode != NOVAQ_PAD_ZEROS && (cg.ph || cg.pw)) || cg.KH != cg.KW ||
       (cg.KH != 3 && cg.KH != 1) || cg.C % CK_C)
     return false;
   ChunkGeom g{};
   g.N = cg.N; g.C = cg.C; g.H = cg.H; g.W = cg.W; g.M = cg.C_out; g.KH = cg.KH; g.KW = cg.KW;
   g.sh = cg.sh; g.sw = cg.sw; g.ph = cg.ph; g.pw = cg.pw; g.OH = cg.OH; g.OW = cg.OW;
-  const auto* wq = static_cast<const uint8_t*>(w);
-  return cg.KH == 3 ? chunk_launch<WT, XT, 9>(x, x_scale, wq, w_scale, ep, y, g, least, stream, rc)
-                    : chunk_launch<WT, XT, 1>(x, x_scale, wq, w_scale, ep, y, g, least, stream, rc);
+  const int wide_least = device_cu_count() / 2;
+  return cg.KH == 3 ? chunk_plan<WT, 9>(g, wide_least, p) : chunk_plan<WT, 1>(g, wide_least, p);
+}
+
+enum class ConvPath { Chunk, Bands, Gather };
+
+// Which path is the fastest for a shape that chunks and bands both take (p, and
+// `blocks` workgroups of `lds` bytes; at most 64 channels), from the three
+// measured on 2700 calls (FP8 and FP4 weights, fp32 and bf16 x, 32 and 64
+// channels to 16 .. 128, maps of 4 x 4 to 125 x 125, 2 to 2048 of them; us):
+//   - small maps whose bands need little LDS, so that all of a launch's are on
+//     the chip together, while a chunked workgroup puts several images, or few of
+//     its pixel slots, through one long chain.  64 -> 32 channels, 1 x 1, 256
+//     maps of 7 x 7: chunks 15.2, bands 8.8, gathered 6.8; 32 -> 32, 3 x 3, 256
+//     maps of 7 x 7 (FP4): 13.8, 8.4, 9.3; 32 -> 128, 3 x 3 / 2, 256 maps of 14
+//     x 14 (FP4): 22.4, 12.8, 13.8.  The gathered kernel is the best of them up
+//     to 64 pixels a CU, for few channels and bands that are not the smallest;
+//   - many workgroups of one chunk and more than 32 output channels: with
+//     nothing to overlap a chunk's load, the larger bands win for FP4 weights and
+//     where 64-channel blocks are a quarter empty or more (32 -> 96, 256 maps of
+//     20 x 20: 27.1 against 19.4; 32 -> 128, 16 maps of 112 x 112, whose chunks
+//     are single rows: 60.0, 49.4; 32 -> 96, 145 maps of 45 x 45: 111.7, 79.7),
+//     and for 1 x 1 windows of narrow x (32 -> 64, 256 maps of 28 x 28, bf16:
+//     19.6, 15.9);
+//   - chunks otherwise: 64 -> 64 on 64 maps of 14 x 14 half the bands' time.
+template <int WT, int XT>
+ConvPath best_path(const ConvGeom& g, const ChunkPlan& p, size_t lds, int64_t blocks) {
+  constexpr bool F32X = XL<XT>::bytes == 4;
+  constexpr size_t KB = 1024;
+  const int64_t cus = device_cu_count(), plane = (int64_t)g.OH * g.OW, wgs = p.blocks();
+  const bool unit = g.sh == 1 && g.sw == 1;
+  const size_t fill = (size_t)blocks * lds / (size_t)cus;  // LDS of a CU's bands
+  bool small = false;
+  if (g.KH == 1)
+    small = unit && plane > 42 && fill <= 40 * KB &&
+            (plane <= 100 ? lds <= 17 * KB : F32X && plane <= 170 && lds <= 14400);
+  else if (unit)
+    small = g.C_out <= 32 && p.g.G >= 3 && plane > 42 && lds <= 28 * KB && fill <= 48 * KB;
+  else if (g.sh == 2 && g.sw == 2)
+    small = plane >= 24 && lds <= 28000 && fill <= 56 * KB;
+  if (small)
+    return g.N * plane <= 64 * cus && g.C_out <= 32 && (unit || lds > 20 * KB) ? ConvPath::Gather
+                                                                             : ConvPath::Bands;
+  if (g.C_out > 32 && unit) {
+    const bool quads = g.W % 4 == 0;
+    if (g.KH == 1) {
+      if (!F32X && quads && wgs >= 6 * cus) return ConvPath::Bands;
+    } else if (g.C == CK_C && (WT == E2M1 || (g.C_out % 64 >= 1 && g.C_out % 64 <= 48))) {
+      // rows of other widths: fp32 ones whose chunks are a quarter empty or more
+      const bool empty = g.N * plane * 4 < (int64_t)3 * 128 * p.g.groups * p.g.bands;
+      if (quads ? (p.g.R == 1 ? wgs >= 3 * cus : lds <= BAND_LDS_FOUR && wgs >= 6 * cus)
+                : F32X && empty && wgs >= 4 * cus)
+        return ConvPath::Bands;
+    }
+  }
+  // (9 x 9 maps fill 81 of the tile's 128 pixels: 32 -> 64, 300 maps, FP4: 14.7, 12.5)
+  if (WT == E2M1 && F32X && g.KH == 3 && unit && g.C == CK_C && g.C_out > 32 && p.g.G == 1 &&
+      plane > 64 && plane < 86)
+    return ConvPath::Bands;
+  return ConvPath::Chunk;
 }
 
 // The gathered path where it takes the shape; returns false otherwise.
@@ -1669,6 +1723,25 @@ bool launch_gather(const uint8_t* x, const float* x_scale, const void* w, const 
   return true;
 }
 
+// Fewer bands than CUs are gathered instead (64 -> 64 channels, 3 x 3, 16 maps of
+// 14 x 14 = 16 bands: 11.2 us, 23.1 in bands), but for more than 32 output
+// channels (the gathered kernel's larger tiles) where bands of little LDS have
+// many pixels all the same (16 -> 48, 48 maps of 28 x 28: 13.8 us gathered, 10.4
+// in bands, on 32 of them 8.7, 10.0; 40 -> 48, 1 x 1, 48 maps: 12.8, 9.2; 8 ->
+// 48, 250 maps of 14 x 14: 14.2, 9.1), and few channels on small maps with a stride of 2 or a 1 x 1
+// window (24 -> 64, 1 x 1, 9 x 9: 10.0, 8.3).  1900 calls of 5 to 48 channels,
+// each way: 64 more than 5% slower than in bands, 7 than gathered; all gathered:
+// 249.
+inline bool few_bands_best(const ConvGeom& g, int taps, size_t lds, int64_t co_blocks) {
+  if (g.C_out <= 32) return false;
+  const int64_t plane = (int64_t)g.OH * g.OW;
+  if (g.N * plane * co_blocks >= (int64_t)112 * device_cu_count() && lds <= BAND_LDS_FOUR &&
+      (taps <= 9 || g.C < 8) && (g.W % 4 == 0 || (g.C <= 24 && plane <= 256)))
+    return true;
+  return g.C <= 24 && lds <= 12 * 1024 && plane <= 100 &&
+         (taps == 1 || (taps == 9 && g.sh == 2 && g.sw == 2));
+}
+
 template <int WT, int XT>
 int launch(const uint8_t* x, const float* x_scale, const void* w, const float* w_scale,
            const Epilogue& ep, void* y, ConvGeom g, hipStream_t stream) {
@@ -1691,27 +1764,31 @@ int launch(const uint8_t* x, const float* x_scale, const void* w, const float* w
   int ipt = 0;
   const bool band = band_geometry<WT>(g, b, band_lds, &ipt, ep.out_dtype);
   const int64_t co_blocks = (g.C_out + CO_TILE - 1) / CO_TILE;
+  const int64_t band_blocks = band ? (int64_t)g.N * b.bands * co_blocks : 0;
   // The chunked path where its workgroups cover an eighth of the CUs (96 -> 70
   // channels, 3 maps of 13 x 17 = 12 workgroups: 17.1 us, gathered 13.2; 64 ->
-  // 64, 16 maps of 14 x 14 = 32: 9.8 against 10.9), but for one chunk of FP4
-  // weights on bands that fill the chip (32 -> 64, 256 maps of 28 x 28: 25.0
-  // us, in bands 23.5).
+  // 64, 16 maps of 14 x 14 = 32: 9.8 against 10.9), and where neither bands nor
+  // the gathered kernel are the better ones (best_path).
+  bool gather = !band || (band_blocks < device_cu_count() &&
+                          !few_bands_best(g, b.taps, band_lds, co_blocks));
   if constexpr (dtype_bits(WT) <= 8) {
-    const bool bands_best = WT == E2M1 && band && band_lds <= BAND_LDS_FOUR && g.C == CK_C &&
-                            b.taps == 9 && g.sh == 1 && g.sw == 1 &&
-                            (int64_t)g.N * b.bands * co_blocks >= 2 * (int64_t)device_cu_count();
-    int rc = NOVAQ_OK;
-    if (!bands_best &&
-        launch_chunk<WT, XT>(x, x_scale, w, w_scale, ep, y, g, device_cu_count() / 8, stream, &rc))
-      return rc;
+    ChunkPlan p;
+    if (plan_chunk<WT>(g, p)) {
+      const ConvPath path = band ? best_path<WT, XT>(g, p, band_lds, band_blocks) : ConvPath::Chunk;
+      if (path == ConvPath::Chunk && p.blocks() >= device_cu_count() / 8) {
+        const auto* wq = static_cast<const uint8_t*>(w);
+        return g.KH == 3 ? chunk_launch<WT, XT, 9>(x, x_scale, wq, w_scale, ep, y, p, stream)
+                         : chunk_launch<WT, XT, 1>(x, x_scale, wq, w_scale, ep, y, p, stream);
+      }
+      if (path != ConvPath::Chunk) gather = path == ConvPath::Gather;
+    }
   }
-  // The gathered path wherever no band fits in LDS, and where bands would
-  // leave CUs idle (64 -> 64 channels, 3 x 3, 16 maps of 14 x 14 = 16 bands:
-  // 11.2 us gathered, 23.1 in bands; 400 bands of 16 -> 48 channels 28.6
-  // against 17.7) or fill a CU with fewer than four workgroups of a large
-  // window's weights (32 -> 64, 5 x 5, 64 maps of 28 x 28: 31.2 against 49.3).
-  if (!band || (int64_t)g.N * b.bands * co_blocks < device_cu_count() ||
-      (band_lds > BAND_LDS_FOUR && b.taps > 9)) {
+  // Gathered as well where a band fills a CU with fewer than four workgroups of
+  // a large window's weights over more than 16 channels (32 -> 64, 5 x 5, 64 maps
+  // of 28 x 28: 31.2 against 49.3; 16 -> 32, 256 maps, bf16 weights: 44.7 against
+  // 37.3, fp32 ones 51.3 against 56.5, at 4 x 4 48.4 against 37.4).
+  if (gather || (band_lds > BAND_LDS_FOUR && b.taps > 9 &&
+                 (g.C > 16 || (WT == F32 && b.taps > 16)))) {
     int rc = NOVAQ_OK;
     if (launch_gather<WT, XT>(x, x_scale, w, w_scale, ep, y, g, stream, &rc)) return rc;
   }

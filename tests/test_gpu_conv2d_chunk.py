@@ -88,3 +88,20 @@ def test_chunked_conv_nan_stays_in_its_windows():
     bad = np.zeros(y.shape, bool)
     bad[2, :, 4:6, 0:2] = True
     assert np.array_equal(np.isnan(y), bad)
+
+
+# (N, C, H, W, C_out, k, stride, padding): 32 or 64 channels that chunks, bands
+# and the gathered kernel all take, each side of the lines between them
+BETWEEN = [
+    (256, 32, 7, 7, 32, 3, 1, 1), (600, 32, 7, 7, 17, 3, 1, 1), (64, 64, 9, 9, 30, 3, 1, 1),
+    (256, 64, 7, 7, 32, 1, 1, 0), (600, 32, 9, 9, 64, 1, 1, 0), (40, 32, 14, 14, 32, 3, 2, 1),
+    (90, 64, 10, 9, 33, 3, 2, 1), (300, 32, 9, 9, 70, 3, 1, 1), (520, 32, 12, 12, 70, 3, 1, 1),
+    (3, 32, 99, 100, 96, 3, 1, 1), (512, 32, 13, 13, 96, 3, 1, 1), (200, 32, 28, 28, 48, 1, 1, 0),
+]
+
+
+@pytest.mark.parametrize("wdt", ["e4m3", "e2m1"])
+@pytest.mark.parametrize("shape", BETWEEN, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
+def test_shapes_that_several_kernels_take(shape, wdt, xdt):
+    test_chunked_conv_exact_operands(shape, wdt, xdt)
