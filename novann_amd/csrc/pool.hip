@@ -792,6 +792,25 @@ inline bool pool_tile_geometry(const PoolGeom& g, PoolTile& t, size_t& lds) {
   return (planes + P - 1) / P <= 0x7FFFFFFF;
 }
 
+// Whether max_pool2d_bwd_kernel's walk, a lane an element, is the faster way all
+// the same: where a plane is a long chain for its one workgroup, the planes are
+// too few to keep the chip busy, and an element's windows cost little to work out
+// again (one window an element: 16 planes of 100 x 100, 3 x 3 / 3, 6.8 us, 9.7 in
+// tiles, 2 x 2 / 3 6.5, 10.8; 4 planes, 5 x 5 / 5 9.9, 12.3; 64 planes of 57 x 58,
+// 2 x 2 / 2 6.7, 7.6; the tiles win from 64 planes of 80 x 80, 3 x 3 / 3: 8.9, 7.5,
+// and up to 29 x 30: 6.9, 3.7.  Four windows an element, 3 x 3 / 2: 4 planes of 80 x
+// 80 14.5, 15.9; of 57 x 58 14.6, 12.9).
+inline bool pool_walk_best(const PoolGeom& g) {
+  const int64_t hw = (int64_t)g.H * g.W, planes = g.N * g.C, cus = device_cu_count();
+  const int64_t taps = (int64_t)g.KH * g.KW;
+  const int64_t windows =
+      (((int64_t)g.KH + g.sh - 1) / g.sh) * (((int64_t)g.KW + g.sw - 1) / g.sw);
+  if (windows == 1)
+    return hw >= std::max<int64_t>(POOL_TILE_ELEMS, 320 * taps) &&
+           planes * hw * std::min<int64_t>(taps, 9) <= 10240 * cus;
+  return hw > 6000 && planes <= cus / 16 && windows * taps <= 36;
+}
+
 // Stages np padded planes from element e0 of x as fp32 bits.
 template <int XT>
 __device__ __forceinline__ void pool_stage(const uint8_t* __restrict__ x, int64_t e0, int np,
@@ -1036,7 +1055,7 @@ int launch_max_bwd(const float* grad, const void* x, float* gi, const PoolGeom& 
   }
   PoolTile t{};
   size_t lds = 0;
-  if (pool_tile_geometry(g, t, lds)) {
+  if (!pool_walk_best(g) && pool_tile_geometry(g, t, lds)) {
     t.vec = reinterpret_cast<uintptr_t>(x) % (4 * EB) == 0 &&
             reinterpret_cast<uintptr_t>(gi) % 16 == 0 && (int64_t)t.P * g.H * g.W % 4 == 0 &&
             g.N * g.C * g.H * (int64_t)g.W % 4 == 0;

@@ -62,3 +62,14 @@ def test_windows_bit_exact(shape, special, mode):
         got = F.max_pool2d_backward(gd, xd, k, s, p, mode).cpu().numpy()
         assert np.array_equal(np.isnan(got), np.isnan(gi))
         assert np.array_equal(got[~np.isnan(gi)].view(np.uint32), gi[~np.isnan(gi)].view(np.uint32))
+
+
+# few large planes: walked an element a lane; one pixel or plane less in tiles
+FEW = [(1, 3, 57, 58, 2, 2, 0), (1, 64, 57, 58, 3, 3, 0), (2, 2, 90, 91, 2, 3, 0),
+       (1, 2, 45, 45, 2, 2, 0), (1, 4, 80, 80, 3, 2, 1), (17, 1, 80, 80, 3, 2, 1)]
+
+
+@pytest.mark.parametrize("shape", FEW, ids=lambda s: "x".join(map(str, s)))
+def test_few_large_planes_bit_exact(shape):
+    for special in (False, True):
+        test_windows_bit_exact(shape, special, "zeros")
