@@ -164,6 +164,14 @@ __global__ __launch_bounds__(256) void c1_tail_kernel(FinishArgs a, const float*
                           cg, (int)(b - a.wb - a.bb), t_lds);
 }
 
+// p[0 .. n) = 0 (p on 16 bytes).
+__global__ __launch_bounds__(256) void zero_kernel(float* __restrict__ p, int64_t n) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+  for (int64_t i = t; i < n / 4; i += step)
+    reinterpret_cast<float4*>(p)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int64_t i = n / 4 * 4 + t; i < n; i += step) p[i] = 0.0f;
+}
+
 // grad_input for strides above 1 and wide paddings, in fp32: a lane makes one
 // input pixel of CT channels.  The taps that reach a pixel are those
 // congruent to its row and column modulo the strides, so a workgroup takes
@@ -172,7 +180,8 @@ __global__ __launch_bounds__(256) void c1_tail_kernel(FinishArgs a, const float*
 // is phases x layers x blocks of pixels).  Per tap and 128 output channels the
 // weights of those channels are decoded once into LDS, times the scale; a lane
 // then loads one grad value an output channel and adds CT products.  A tap
-// outside grad is skipped, not multiplied by zero.
+// outside grad is skipped, not multiplied by zero.  by_tap: only the phases
+// that a tap reaches are run, on a zeroed grad_input.
 //
 // Bound by the LDS pipe (four broadcast reads to 16 products; two pixels a
 // lane need a select a product for the taps only one of them has: 271 us
@@ -188,14 +197,27 @@ __global__ __launch_bounds__(256) void dinput_phase_kernel(const float* __restri
                                                           const uint8_t* __restrict__ w,
                                                           const float* __restrict__ w_scale,
                                                           float* __restrict__ gi, BwdGeom g,
-                                                          int blocks, int layers) {
+                                                          int blocks, int layers, int by_tap) {
   constexpr int LANES = SPLIT ? 64 : 256;  // lanes on different pixels
   __shared__ __attribute__((aligned(16))) float wt[DI_CO * CT];
   const int phase = (int)blockIdx.x / (blocks * layers), rest = (int)blockIdx.x - phase * blocks * layers;
   const int layer = rest / blocks;
   // pixels (h0 + sh i, w0 + sw j); taps a, a + sh, ... and b, b + sw, ...
-  const int h0 = phase / min(g.sw, g.W), w0 = phase - h0 * min(g.sw, g.W);
-  const int a = (h0 + g.ph) % g.sh, b = (w0 + g.pw) % g.sw;
+  int h0, w0, a, b;
+  if (by_tap) {  // the phases that a tap reaches, numbered by their first one
+    a = phase / g.KW;
+    b = phase - a * g.KW;
+    h0 = a - g.ph % g.sh;
+    w0 = b - g.pw % g.sw;
+    h0 += h0 < 0 ? g.sh : 0;
+    w0 += w0 < 0 ? g.sw : 0;
+    if (h0 >= g.H || w0 >= g.W) return;  // the whole workgroup
+  } else {
+    h0 = phase / min(g.sw, g.W);
+    w0 = phase - h0 * min(g.sw, g.W);
+    a = (h0 + g.ph) % g.sh;
+    b = (w0 + g.pw) % g.sw;
+  }
   const int Hp = (g.H - 1 - h0) / g.sh + 1, Wp = (g.W - 1 - w0) / g.sw + 1;
   const int64_t total = (int64_t)g.N * Hp * Wp;
   const int64_t first = (int64_t)(rest - layer * blocks) * LANES;
@@ -1288,9 +1310,18 @@ int launch_dinput(const float* grad, const void* w, const void* wf, const float*
   // the blocks of the largest phase; 16 channels a layer, 8 for the few of a
   // first layer
   const int64_t pixels = (int64_t)g.N * ((g.H + (int64_t)g.sh - 1) / g.sh) * ((g.W + (int64_t)g.sw - 1) / g.sw);
-  const int64_t phases = (int64_t)std::min(g.sh, g.H) * std::min(g.sw, g.W);
+  const int64_t all = (int64_t)std::min(g.sh, g.H) * std::min(g.sw, g.W);
   const int ct = g.C > 8 ? 16 : 8;
   const int64_t layers = (g.C + ct - 1) / ct;
+  // Strides far above the window leave most phases without a tap and with few
+  // pixels each; where their workgroups are many, grad_input is zeroed and the
+  // taps' phases alone are run (1 channel, 3 x 3 / 300, one 512 x 512 image: 90000
+  // phases, 122 us as they are, 18.6 so; 64 channels, 3 x 3 / 50, two of 64 x 64:
+  // 26.2, 18.9; with fewer workgroups the second launch costs more: 16 channels, 3 x
+  // 3 / 50, one of 100 x 100 = 2500 workgroups 15.7, 18.5).
+  const bool by_tap = g.KH <= g.sh && g.KW <= g.sw && all >= (int64_t)64 * g.KH * g.KW &&
+                      all * layers >= 8192;
+  const int64_t phases = by_tap ? (int64_t)g.KH * g.KW : all;
   // 256 pixels a workgroup while that gives every CU four workgroups
   const bool split = (pixels + 255) / 256 * layers * phases < 4 * (int64_t)device_cu_count();
   const int64_t per = split ? 64 : 256, blocks = (pixels + per - 1) / per;
@@ -1298,8 +1329,15 @@ int launch_dinput(const float* grad, const void* w, const void* wf, const float*
     return NOVAQ_EINVAL;
   auto kern = split ? (ct == 16 ? dinput_phase_kernel<WT, 16, true> : dinput_phase_kernel<WT, 8, true>)
                     : (ct == 16 ? dinput_phase_kernel<WT, 16, false> : dinput_phase_kernel<WT, 8, false>);
+  if (by_tap) {
+    const int64_t n = (int64_t)g.N * g.C * g.H * g.W, most = 16 * (int64_t)device_cu_count();
+    const unsigned zb = (unsigned)std::min<int64_t>((n / 4 + 255) / 256 + 1, most);
+    hipLaunchKernelGGL(zero_kernel, dim3(zb), dim3(256), 0, stream, gi, n);
+    const int rc = check_launch();
+    if (rc != NOVAQ_OK) return rc;
+  }
   hipLaunchKernelGGL(kern, dim3((unsigned)(blocks * layers * phases)), dim3(256), 0, stream, grad,
-                     static_cast<const uint8_t*>(w), w_scale, gi, g, (int)blocks, (int)layers);
+                     static_cast<const uint8_t*>(w), w_scale, gi, g, (int)blocks, (int)layers, by_tap);
   return check_launch();
 }
 

@@ -30,6 +30,11 @@ SHAPES = [
     (1, 3, 6, 6, 7, 3, 3, (1, 1), (4, 3)),         # stride 1, padding past the window
     (65, 8, 4, 4, 130, 3, 3, (2, 2), (1, 1)),      # 260 pixels a phase
     (70, 130, 18, 18, 32, 3, 3, (2, 2), (1, 1)),   # many workgroups of 256 pixels
+    # the taps' phases alone: one pixel each and a few, taps on the padding, pixels
+    # past the image
+    (3, 20, 70, 80, 6, 2, 3, (70, 80), (0, 0)),
+    (1, 3, 131, 127, 5, 3, 2, (90, 100), (1, 0)),
+    (2, 130, 33, 34, 7, 3, 3, (40, 32), (2, 7)),
 ]
 
 
