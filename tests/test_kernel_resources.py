@@ -35,14 +35,9 @@ def test_no_vector_register_spills(res):
     assert not spilled, list(spilled)[:5]
 
 
-def test_scratch_only_where_expected(res):
-    # one kernel uses scratch by design, nothing else: the guarded edge-tile
-    # Linear kernel (one workgroup per CU, 110 KB of LDS) spills 14 scalar
-    # registers
-    for name, r in res.items():
-        if not r.get("scratch", 0):
-            continue
-        assert "linear_kernel" in name and r.get("vgpr_spill", 0) == 0, (name, r)
+def test_no_kernel_uses_scratch(res):
+    scratch = {n: r for n, r in res.items() if r.get("scratch", 0)}
+    assert not scratch, list(scratch)[:5]
 
 
 def test_band_convolution_keeps_four_workgroups_per_cu(res):
