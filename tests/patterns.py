@@ -30,7 +30,7 @@ def random_f32_bits(n: int, seed: int) -> np.ndarray:
 
 
 def config1_tensor(seed: int = 1, shape=(4096, 4096)) -> np.ndarray:
-    """BASELINE config [1]: 90% N(0,1), 10% specials (+-0, +-Inf, NaNs,
+    """Special values: 90% N(0,1), 10% specials (+-0, +-Inf, NaNs,
     subnormal-E4M3 neighbourhood k*2^-9 +- ulp and ties, and an overflow band
     448 .. fp32 max including 464 and 480)."""
     rng = np.random.default_rng(seed)
@@ -75,7 +75,7 @@ def config1_tensor(seed: int = 1, shape=(4096, 4096)) -> np.ndarray:
 
 
 def config2_tensor(n: int, seed: int = 2) -> np.ndarray:
-    """BASELINE config [2]: random sign, |x| log-uniform in [2^-20, 2^20]."""
+    """Wide range: random sign, |x| log-uniform in [2^-20, 2^20]."""
     rng = np.random.default_rng(seed)
     mag = np.exp2(rng.uniform(-20.0, 20.0, size=n)).astype(np.float32)
     sgn = np.where(rng.random(n) < 0.5, -1.0, 1.0).astype(np.float32)
@@ -83,7 +83,7 @@ def config2_tensor(n: int, seed: int = 2) -> np.ndarray:
 
 
 def config3_tensor(n: int, seed: int = 3) -> np.ndarray:
-    """BASELINE config [3]: N(0,1) divided by amax/6 (so the tensor spans the
+    """FP4 range: N(0,1) divided by amax/6 (so the tensor spans the
     E2M1 range), with 5% of the entries replaced by exact E2M1 RNE ties."""
     rng = np.random.default_rng(seed)
     x = rng.standard_normal(n, dtype=np.float32)

@@ -5,8 +5,8 @@ plus the layout kernels they are built from.
 Tolerances: transposes are bit-exact (codes permuted; fp32 -> bf16 / fp16 by
 the oracle's cast); the column sum is an fp32 sum, within 1e-5 relative of
 fp64; the gradients are normwise max|g - r| / max|r| <= 1e-2 against fp64 on
-the same fp32 inputs and the dequantized weight (the BASELINE tolerance of the
-forward product)."""
+the same fp32 inputs and the dequantized weight (the tolerance of the forward
+product)."""
 import numpy as np
 import pytest
 import torch
@@ -116,9 +116,9 @@ def weight_of(w, wdt):
 
 @pytest.mark.parametrize("wdt", ["e4m3", "e5m2", "e2m1", "f32"])
 @pytest.mark.parametrize("N,D_in,D_out", [
-    (256, 512, 256),     # whole tiles: the fast forward kernels on both products
-    (2048, 1024, 512),
-    (64, 96, 40),        # ragged: guarded kernels
+    (256, 512, 256),     # whole tiles
+    (2048, 1024, 512),   # grad_input on the 128 x 256-tile kernels
+    (64, 96, 40),        # ragged
     (33, 70, 46),
 ])
 def test_linear_backward_vs_oracle(wdt, N, D_in, D_out):
@@ -144,15 +144,15 @@ def bf16_round(a):
 
 
 # D_out % 128, D_in % 256, N % 64: the weight gradient reads grad and x in
-# place (transposing LDS reads); tile counts 1, 9 (not a multiple of 8) and 16,
-# and config [4]'s weight (256 x 256 tiles, one per CU)
+# place, on the split-K kernel for tile counts 1, 9 and 16 and through transposing
+# LDS reads for a 4096 x 4096 weight (256 x 256 tiles, one per CU)
 @pytest.mark.parametrize("N,D_in,D_out", [(64, 256, 128), (128, 768, 384), (192, 1024, 512),
                                           (1024, 4096, 4096)])
 def test_weight_gradient_in_place_product(N, D_in, D_out):
     """grad_weight = grad^T x equals the fp64 product of the bf16-rounded
     operands up to fp32 summation error (1e-5 normwise): an index or layout
-    slip in the transposing reads is far outside that; likewise grad_input on
-    the bf16 copy of grad that product stores, and the fused bias sum."""
+    slip in the K-major reads is far outside that; likewise grad_input on grad
+    rounded to bf16, and the fused bias sum."""
     print(f"grad_weight in place N={N} D_in={D_in} D_out={D_out}", flush=True)
     rng = np.random.default_rng(N * 7 + D_in)
     x = rng.standard_normal((N, D_in)).astype(np.float32)
@@ -164,7 +164,7 @@ def test_weight_gradient_in_place_product(N, D_in, D_out):
     g16 = bf16_round(g).astype(np.float64)
     assert normwise(gw.cpu().numpy(), g16.T @ bf16_round(x).astype(np.float64)) <= 1e-5
     assert normwise(gb.cpu().numpy(), g.astype(np.float64).sum(0, keepdims=True)) <= 1e-5
-    # grad_input multiplies the bf16 grad the weight-gradient product left behind
+    # grad_input multiplies grad rounded to bf16
     assert normwise(gi.cpu().numpy(), g16 @ wdeq) <= 1e-5
     lib = _lib.load()
     assert lib.novaq_linear_backward_workspace(N, D_in, D_out, 3) < \
@@ -175,10 +175,9 @@ def test_weight_gradient_in_place_product(N, D_in, D_out):
                                           (384, 768, 1024, "e4m3"), (128, 512, 256, "e2m1")])
 def test_input_gradient_on_weight_codes_in_place(N, D_in, D_out, dt):
     """grad_input = bf16(grad) @ (s * dec(W)) with W's FP8 codes read in their
-    stored (D_out, D_in) layout through transposing LDS reads, and the fp32
-    grad rounded to bf16 while staged: within 1e-5 normwise of the fp64
-    product, with and without grad_weight asked for; E2M1 takes the transposed
-    copy.  The in-place shapes need no workspace (NULL is accepted)."""
+    stored (D_out, D_in) layout, and the fp32 grad rounded to bf16 while loaded:
+    within 1e-5 normwise of the fp64 product, with and without grad_weight asked
+    for.  FP8 weights in whole tiles need no workspace (NULL is accepted)."""
     print(f"grad_input in place N={N} D_in={D_in} D_out={D_out} {dt}", flush=True)
     rng = np.random.default_rng(N + D_in * 3 + D_out)
     x = rng.standard_normal((N, D_in)).astype(np.float32)
@@ -204,7 +203,7 @@ def test_input_gradient_on_weight_codes_in_place(N, D_in, D_out, dt):
     torch.cuda.synchronize()
     assert normwise(gi2.cpu().numpy(), ref) <= 1e-5
     # FP8 W: no workspace (W's codes and the fp32 grad read in place); E2M1:
-    # W^T, then the bf16 grad the weight-gradient product leaves
+    # room for W^T and the bf16 grad that products of more tiles take
     grad_bytes = -(-N * D_out * 2 // 256) * 256
     wt_bytes = -(-D_in * D_out * 4 // 8 // 256) * 256
     assert nbytes == (wt_bytes + grad_bytes if dt == "e2m1" else 0)

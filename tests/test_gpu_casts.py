@@ -103,7 +103,7 @@ def test_scaled_quantize_and_dequantize(dt, scale):
 
 
 def test_config1_e4m3_roundtrip_bit_exact():
-    """BASELINE config [1]: 4096x4096 fp32 with 10% specials -> E4M3 -> fp32."""
+    """4096x4096 fp32 with 10% specials -> E4M3 -> fp32."""
     x = config1_tensor()
     bits = x.view(np.uint32).reshape(-1)
     q = quant.cast(to_dev(bits, O.F32), "e4m3")
@@ -116,7 +116,7 @@ def test_config1_e4m3_roundtrip_bit_exact():
 
 
 def test_config2_sweep_full_size_bit_exact():
-    """BASELINE config [2] at full size: 2^28 fp32 -> {f16, bf16} -> fp32 and
+    """2^28 fp32 -> {f16, bf16} -> fp32 and
     per-tensor amax-scaled {E4M3, E5M2} -> fp32, all bit-compared."""
     n = 1 << 28
     x = config2_tensor(n)
@@ -148,7 +148,7 @@ def test_config2_sweep_full_size_bit_exact():
 
 @pytest.mark.parametrize("n", [1 << 26, (1 << 26) - 3])
 def test_config3_fp4_pack_unpack_bit_exact(n):
-    """BASELINE config [3]: 2^26 elements (and an odd size), pack with the
+    """2^26 elements (and an odd size), pack with the
     per-tensor amax/6 scale, unpack; the packed bytes are bit-compared."""
     x = config3_tensor(n)
     xd = to_dev(x.view(np.uint32), O.F32)

@@ -2,7 +2,7 @@
 numpy im2col restatement of novann/functional.py:275-385).
 
 Tolerance: normwise max|y - r| / max|r| <= 1e-2 against fp64 on the same fp32
-input and the dequantized fp32 weights (BASELINE north star)."""
+input and the dequantized fp32 weights."""
 import numpy as np
 import pytest
 import torch
@@ -120,7 +120,7 @@ def test_shapes_and_modes_vs_oracle(wdt, mode, case):
 
 @pytest.mark.parametrize("case", [
     # (N, C, H, W, KH, KW, ph, pw, mode)
-    (4, 32, 28, 28, 3, 3, 1, 1, "zeros"),     # config [5] conv1's input gradient, 4 images
+    (4, 32, 28, 28, 3, 3, 1, 1, "zeros"),     # a one-channel layer's input gradient, 4 images
     (2, 37, 13, 20, 2, 5, 0, 2, "reflect"),   # C no multiple of 8
     (3, 8, 30, 8, 7, 7, 3, 3, "circular"),    # 7 x 7, rows wider than the image's 8 columns
     (1, 6, 70, 4, 3, 1, 1, 0, "replicate"),   # narrow rows: many rows per band
@@ -146,7 +146,7 @@ def test_one_output_channel_exact_operands(case):
 
 
 def test_config5_mnist_two_layers():
-    """BASELINE config [5]: x (256, 1, 28, 28) U[0,1]; conv1 1->32 and conv2
+    """x (256, 1, 28, 28) U[0,1]; conv1 1->32 and conv2
     32->64, 3x3 / stride 1 / pad 1, Kaiming-normal weights in E2M1 with
     per-tensor scale, bias zero, conv2 applied to conv1's fp32 output."""
     rng = np.random.default_rng(5)
@@ -178,8 +178,8 @@ def test_config5_mnist_two_layers():
     # input rounded to bf16, W decoded exactly): fp32 summation error only
     e1 = error_report(y1h, O.conv2d_f64(bf16_round(x), w1d, (1, 1), (1, 1)).astype(np.float64))
     e2 = error_report(y2h, O.conv2d_f64(bf16_round(y1h), w2d, (1, 1), (1, 1)).astype(np.float64))
-    print(f"config [5] conv1 vs fp32-input fp64: {rep1}; exact-operand: {e1}", flush=True)
-    print(f"config [5] conv2 vs fp32-input fp64: {rep2}; exact-operand: {e2}", flush=True)
+    print(f"conv1 vs fp32-input fp64: {rep1}; exact-operand: {e1}", flush=True)
+    print(f"conv2 vs fp32-input fp64: {rep2}; exact-operand: {e2}", flush=True)
     assert e1["normwise"] <= 1e-5 and e2["normwise"] <= 1e-5, (e1, e2)
 
 

@@ -3,7 +3,7 @@ the CPU restatement of Conv2d.backward and _col2im
 (novann/layers/convolutional/conv2d.py:117-148, 179-207).
 
 Tolerance: normwise max|g - r| / max|r| <= 1e-2 against fp64 on the same fp32
-grad and input and the dequantized weight (the BASELINE tolerance of the
+grad and input and the dequantized weight (the tolerance of the
 forward products).  grad_bias is an fp32 sum, so it is held to 1e-5."""
 import numpy as np
 import pytest
@@ -165,7 +165,7 @@ C1_GEOMETRIES = [
     (3, 9, 20, 40, 3, 5, (1, 2), "reflect"),      # 15 taps, three channel tiles
     (1, 17, 39, 64, 4, 4, (2, 2), "replicate"),   # 16 taps, 40-pixel rows (two k-steps a row)
     (2, 7, 8, 33, 2, 3, (0, 1), "circular"),      # a partial last channel tile
-    (5, 30, 28, 32, 3, 3, (1, 1), "zeros"),       # config [5] conv1's shape, 5 images
+    (5, 30, 28, 32, 3, 3, (1, 1), "zeros"),       # one input channel, 5 images
 ]
 
 

@@ -1,11 +1,12 @@
 """Fused epilogues of the forward products on the GPU (through the C ABI).
 
 Bit-exact checks: the epilogue's fp32 steps equal the oracle's fp32 restatement
-applied to the unfused kernel output (every Linear and Conv2d kernel path);
+applied to the unfused kernel output (here the shapes of few tiles and bands;
+test_gpu_linear_tiles.py and test_gpu_conv2d_band.py have the others);
 bf16 / f16 / FP8 stores equal the oracle cast of those fp32 values; the output
 amax equals max |v|.  Reference-path check: conv / linear -> eval BatchNorm
 (fp64, the reference's formula) -> ReLU within normwise 1e-2 of the fused
-result (the BASELINE tolerance of the products)."""
+result (the tolerance of the products)."""
 import ctypes
 
 import numpy as np
@@ -146,10 +147,10 @@ def rounding_classes(rng):
 
 @pytest.mark.parametrize("hw", [4, 3])
 def test_bf16_stores_round_every_class(hw):
-    """bf16 stores of the convolution's epilogue (staged through LDS when
-    rows pack into 8-byte pieces, hw = 4; the lanes' own stores otherwise)
-    equal the oracle's cast for every rounding class: with x = 0 each output
-    channel is its bias, so the bias vector feeds the encoder chosen values."""
+    """bf16 stores of the convolution's epilogue (runs of four pixels, hw = 4, and
+    single ones) equal the oracle's cast for every rounding class: with x = 0 each
+    output channel is its bias, so the bias vector feeds the encoder chosen
+    values."""
     print(f"bf16 store rounding hw={hw}", flush=True)
     rng = np.random.default_rng(17)
     bias = rounding_classes(rng)
@@ -165,12 +166,13 @@ def test_bf16_stores_round_every_class(hw):
 
 
 LINEAR_CASES = [
-    ("e4m3", 256, 512, 256),   # linear_pingpong_kernel
-    ("e2m1", 128, 256, 512),   # linear_wide_kernel, FP4
-    ("bf16", 128, 128, 256),   # linear_pipe_kernel
-    ("f16", 128, 64, 128),     # linear_pipe_kernel, 128-wide tiles
-    ("e5m2", 33, 70, 46),      # linear_kernel (ragged)
-    ("f32", 64, 96, 40),       # linear_kernel (fp32 weights)
+    # linear_split_kernel: 32 x 32 tiles, rows read by quads of lanes (K >= 512) or not
+    ("e4m3", 256, 512, 256),
+    ("e2m1", 128, 256, 512),
+    ("bf16", 128, 128, 256),
+    ("f16", 128, 64, 128),
+    ("e5m2", 33, 70, 46),      # ragged
+    ("f32", 64, 96, 40),       # fp32 weights
 ]
 
 
@@ -188,8 +190,8 @@ def test_linear_epilogue_bit_exact(wdt, N, D_in, D_out):
 
 CONV_CASES = [
     # wdt, (N, C, H, W), C_out, (KH, KW), stride, pad, mode
-    ("e2m1", (3, 8, 12, 12), 16, (3, 3), (1, 1), (1, 1), "zeros"),     # band, K9
-    ("e2m1", (2, 32, 28, 28), 64, (3, 3), (1, 1), (1, 1), "zeros"),   # band, config [5] conv2's bands
+    ("e2m1", (3, 8, 12, 12), 16, (3, 3), (1, 1), (1, 1), "zeros"),    # gathered: few bands
+    ("e2m1", (2, 32, 28, 28), 64, (3, 3), (1, 1), (1, 1), "zeros"),   # gathered: few chunks too
     ("e4m3", (2, 5, 10, 11), 20, (5, 5), (1, 1), (2, 2), "reflect"),   # band, generic regroup
     ("bf16", (2, 4, 9, 9), 70, (3, 3), (2, 2), (1, 1), "replicate"),  # band, 2 co blocks
     ("e5m2", (2, 65, 7, 7), 24, (3, 3), (1, 1), (1, 1), "circular"),  # conv2d_kernel (C > 64)

@@ -54,7 +54,7 @@ ALIGNED_ROWS = [  # fp32, zeros, stride 1, W and OW multiples of 4: aligned-chun
     (2, 2, 9, 8, 3, 7, 1, 3),    # 7 wide, every shift
     (1, 3, 6, 8, 5, 5, 2, 4),    # pw = 4: the first chunk wholly left of the image
     (3, 1, 4, 4, 2, 1, 0, 0),    # rows of a single chunk
-    (2, 4, 28, 28, 3, 3, 1, 1),  # config [5]'s conv2 geometry, small batch
+    (2, 4, 28, 28, 3, 3, 1, 1),  # 32 -> 64 layer's geometry, small batch
 ]
 
 
@@ -142,9 +142,9 @@ def test_reference_conv2d_layer_flow_on_the_extras():
 
 
 def test_config5_conv2_column_matrix_full_size():
-    """config [5]'s conv2 input (256, 32, 28, 28): the 288 x 200704 column
+    """The input of 32 -> 64 channels (256, 32, 28, 28): the 288 x 200704 column
     matrix (231 MB) the reference materialises, bit for bit."""
-    print("im2col config [5] conv2 (231 MB)", flush=True)
+    print("im2col 32 channels of 28 x 28 (231 MB)", flush=True)
     rng = np.random.default_rng(55)
     x = rng.standard_normal((256, 32, 28, 28)).astype(np.float32)
     col = F.im2col(torch.from_numpy(x).cuda(), 3, 1, 1, "zeros")

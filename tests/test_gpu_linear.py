@@ -1,9 +1,13 @@
 """Quantized Linear on the GPU vs the CPU oracle (y = x @ (s*dec(Wq))^T + b).
 
-Tolerance: normwise max|y - r| / max|r| <= 1e-2 against
-the fp64 product of the same fp32 inputs and the dequantized fp32 weights.
-The identity-input case is bit-exact: it routes every weight code through the
-in-kernel decode and the MFMA lane layout unchanged."""
+Tolerance: normwise max|y - r| / max|r| <= 1e-2 against the fp64 product of the
+same fp32 inputs and the dequantized fp32 weights.  The identity-input case is
+bit-exact: it routes every weight code through the in-kernel decode and the MFMA
+lane layout unchanged.
+
+Products of at most CUs / 8 tiles of 128 x 256 run on the split-K kernel, so the
+small shapes here are its; the kernels of 128-row tiles have the same checks in
+test_gpu_linear_tiles.py."""
 import numpy as np
 import pytest
 import torch
@@ -60,11 +64,8 @@ def valid_codes(wdt):
 @pytest.mark.parametrize("K,N", [(256, 320), (256, 512), (192, 512), (256, 384)],
                          ids=["edge-tiles", "wide-k", "staged-256", "staged-128"])
 def test_identity_input_reproduces_dequantized_weights_exactly(wdt, scale, K, N):
-    """x = I: y[i, j] = s * dec(W[j, i]) exactly, for every finite code.  The
-    shapes reach each kernel: guarded edge tiles (N % 128 != 0), the K-block
-    kernels for N % 256 == 0, K % 128 == 0 (ping-pong for FP8, wide for FP4)
-    and the staged-decode kernel at both tile widths (K % 128 != 0;
-    N % 256 != 0)."""
+    """x = I: y[i, j] = s * dec(W[j, i]) exactly, for every finite code, over whole
+    and partial tiles of the split-K kernel."""
     rng = np.random.default_rng(1)
     vals = valid_codes(wdt)
     nib = vals[rng.integers(0, vals.size, size=N * K)]
@@ -120,9 +121,8 @@ def test_ragged_shapes_vs_oracle(wdt, M, N, K, with_bias):
                                    (256, 384, 192), (128, 256, 1024), (128, 256, 384),
                                    (256, 768, 640)])
 def test_whole_tile_shapes_vs_oracle(wdt, M, N, K):
-    """Shapes that take the guard-free kernels (M % 128, N % 128, K % 64 == 0):
-    ping-pong (FP8) / wide-K (FP4) when N % 256 and K % 128 are 0,
-    staged-decode at tile width 256 or 128 otherwise and for 16-bit weights."""
+    """Whole tiles of 128 rows, 128 columns and 64 K, too few of them for the
+    kernels of such tiles: the split-K kernel's whole tiles."""
     rng = np.random.default_rng(M + N + K)
     x = rng.standard_normal((M, K)).astype(np.float32)
     w = (rng.standard_normal((N, K)) * np.sqrt(2.0 / K)).astype(np.float32)
@@ -154,8 +154,8 @@ def test_unquantized_weight_dtypes(wdt):
 
 
 def test_config4_full_size():
-    """BASELINE config [4]: x (2048, 4096) N(0,1), W (4096, 4096) Kaiming-normal
-    -> E4M3 with per-tensor amax scale, b = 0."""
+    """x (2048, 4096) N(0,1), W (4096, 4096) Kaiming-normal -> E4M3 with
+    per-tensor amax scale, b = 0."""
     rng = np.random.default_rng(4)
     M, K, N = 2048, 4096, 4096
     x = rng.standard_normal((M, K), dtype=np.float32)
@@ -175,8 +175,8 @@ def test_config4_full_size():
     # to bf16, W decoded exactly): only fp32 summation error is left, so a
     # staging or ordering slip that costs even a few 1e-4 fails here
     exact = error_report(yh, bf16_round(x).astype(np.float64) @ wdeq.T)
-    print(f"config [4] vs fp32-input fp64 product: {rep}", flush=True)
-    print(f"config [4] vs exact-operand fp64 product: {exact}", flush=True)
+    print(f"full size vs fp32-input fp64 product: {rep}", flush=True)
+    print(f"full size vs exact-operand fp64 product: {exact}", flush=True)
     assert exact["normwise"] <= 1e-5, exact
     # quantized weights themselves are the oracle's, bit for bit
     s = O.scale_from_amax(O.amax(w), O.E4M3)
@@ -383,12 +383,12 @@ def test_misaligned_device_views_are_copied_not_refused():
 
 @pytest.mark.parametrize("wdt", ["e4m3", "e5m2"])
 def test_longest_k_one_hot_rows(wdt):
-    """K = 2^21, the longest K the K-block kernels take, forward (W rows of 2
+    """K = 2^21 over few tiles, on the split-K kernel, forward (W rows of 2
     MiB) and backward grad_input (W read in its [K][N] layout): every row of x
     (of grad) is one-hot at a K index spread over the whole range, the first
     and the last included, so y[i, :] = s * dec(W[:, k_i]) (grad_input[i, :]
-    = s * dec(W[k_i, :])) exactly -- the offsets of the last K blocks, near
-    the top of the 31-bit buffer ranges, are exercised."""
+    = s * dec(W[k_i, :])) exactly -- every wave's share of K and its largest
+    offsets are exercised."""
     M, N, K = 128, 256, 1 << 21
     print(f"longest K one-hot {wdt}", flush=True)
     g = torch.Generator(device="cuda")

@@ -49,7 +49,7 @@ def grads(rng, shape):
 
 GEOMS = [
     ((2, 3, 6, 6), (2, 2), (2, 2), (0, 0), "zeros"),        # the reference's gradient check
-    ((256, 64, 28, 28), (2, 2), (2, 2), (0, 0), "zeros"),   # config [5]-sized activations
+    ((256, 64, 28, 28), (2, 2), (2, 2), (0, 0), "zeros"),   # a 28 x 28 layer at batch 256
     ((2, 4, 5, 5), (3, 3), (1, 1), (1, 1), "zeros"),        # overlapping windows
     ((2, 3, 9, 11), (3, 2), (2, 1), (2, 1), "reflect"),
     ((1, 5, 7, 6), (2, 3), (1, 2), (1, 0), "replicate"),

@@ -191,7 +191,7 @@ def test_cast_rejects_quantized_to_quantized():
 
 
 def test_config1_tensor_holds_every_special():
-    """BASELINE config [1]'s specials really occur: signed zeros, both
+    """The special-value tensor's specials really occur: signed zeros, both
     infinities, quiet and signalling NaNs of both signs, values past +-448
     (464 and 480 exactly), E4M3-subnormal neighbours and fp32 subnormals."""
     from tests.patterns import config1_tensor

@@ -53,9 +53,9 @@ def inputs(geo, seed):
     return g, x, wq, torch.tensor([s], dtype=torch.float32, device="cuda")
 
 
-# config [5]'s conv2 at batch 256 (30.8 MB of the 32 MiB scratch), then a
+# 32 -> 64 channels of 28 x 28 at batch 256 (30.8 MB of the 32 MiB scratch), then a
 # smaller, differently shaped call (stride 2, reflect: the general kernels),
-# then config [5]'s conv1 (one input channel: the one-input-channel kernels)
+# then 1 -> 32 channels (one input channel: the one-input-channel kernels)
 CALLS = [(256, 32, 28, 28, 64, 3, 1, 1, "zeros"), (3, 5, 11, 9, 7, 3, 2, 1, "reflect"),
          (256, 1, 28, 28, 32, 3, 1, 1, "zeros")]
 
