@@ -349,14 +349,15 @@ size_t novaq_linear_backward_workspace(int64_t N, int64_t D_in, int64_t D_out, i
  *   grad_bias   (D_out)       = grad summed over the N rows
  * Replaces: Linear.backward (novann/layers/linear/linear.py:85-108).  Any of
  * the three outputs may be NULL (not computed).  The products run on bf16
- * MFMA with fp32 accumulation on grad and x rounded to bf16.  For FP8 w_q at
- * whole-tile shapes (among other limits D_out % 128, D_in % 256 and N % 128
- * are 0) grad_input reads w_q's codes and the fp32 grad in place and
- * grad_weight reads grad and x in place; other shapes go through transposed
- * copies in the workspace (w_q's codes, exact; grad and x in bf16).  The
- * whole condition is the one novaq_linear_backward_workspace() evaluates:
- * when it returns 0, no workspace is needed, whichever gradients are asked
- * for.  grad_bias sums in a fixed order that depends on the shape and on the
+ * MFMA with fp32 accumulation on grad and x rounded to bf16.  Most shapes
+ * read grad, x and w_q's codes in place.  The workspace holds the transposed
+ * codes of E2M1 and 16-bit w_q (exact) where grad_input's product fills the
+ * device with large tiles, grad in bf16 beside them, and bf16 copies of grad
+ * and x transposed for fewer than 4 features.  What the query returns is
+ * enough for whichever gradients are asked for, and 0 means that none is
+ * needed: FP8 w_q in whole tiles (among other limits D_out % 128, D_in % 256
+ * and N % 128 are 0).  It does not depend on the device, and for other
+ * shapes it may be more than the call comes to use.  grad_bias sums in a fixed order that depends on the shape and on the
  * device's CU count (the tile size the weight-gradient product picks), so it
  * is bit-reproducible per device and shape, not across them.  workspace:
  * device memory of novaq_linear_backward_workspace() bytes (16-byte aligned;

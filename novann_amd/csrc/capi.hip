@@ -33,11 +33,13 @@ int device_cu_count() {
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Workspace of novaq_linear_backward: none when grad_input reads W's codes in
-// place (and the fp32 grad, rounding it while staging); otherwise W^T in W's
-// format, then grad in bf16 (at gyt) where the in-place weight-gradient
-// product takes the shape, else grad^T (bf16, at gyt) and x^T (bf16, at xt);
-// each part 256-byte aligned.
+// Workspace of novaq_linear_backward: none for FP8 codes in whole tiles;
+// otherwise W^T in W's format, then (at gyt) grad in bf16 or grad^T in bf16 and,
+// unless the shape is whole tiles of the weight-gradient product, x^T in bf16 (at
+// xt); each part 256-byte aligned.  It holds the parts of every way that the
+// products below may go on any device: W^T and the bf16 grad only where by_wt is
+// set there, grad^T and x^T only without `split` (under 4 features, never whole
+// tiles).  FP8 codes of other shapes use none of it.
 struct LinearBwdWs {
   size_t wt, gyt, xt, total;
   bool tn, wn;

@@ -39,7 +39,11 @@
 // Measured (E4M3 W 4096 x 4096, fp32 x, warm MALL; the guarded 128 x 256-tile
 // kernel it replaced in brackets): 1 row 6.8 us (296), 16 rows 8.4 (306), 64
 // rows 15.7 (342), 14.6 with FP4 W, 9.6 with bf16 x too; 500 x 1024 x 1024 12.6
-// (120); 333 x 777 x 1111 16.8 (277).
+// (120); 333 x 777 x 1111 16.8 (277).  Large products that the tile kernels' ragged
+// forms cannot read run here too: fp32 W 2048 x 4096 x 4096 458 (672), E4M3 W 2000
+// x 4095 x 4096 476 (1339), FP4 W 2048 x 4080 x 4096 277 (868), E4M3 x and W 2000
+// x 4096 x 4096 124 (355).  (The 1 row kernel is 7.4 to 7.6 us in a kernel trace,
+// which adds to short ones; 6.8 between events over a run of launches.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -675,7 +679,12 @@ int split_launch(const uint8_t* x, const float* x_scale, int64_t M, int64_t K, c
     // against 7.3), 2048 K over 16 waves (1024: 5.0, 4.5), and with one
     // workgroup a CU 512 K over 8 (128 x 256 x 256: 5.5, 4.8; 64 x 2048 x 513:
     // 6.0, 8.3), with more 1024 K without a rest (1000 x 500 x 784: 15.2, 11.4;
-    // 500 x 1024 x 1024: 8.9, 9.4) or 2048.
+    // 500 x 1024 x 1024: 8.9, 9.4) or 2048.  Over 3990 products of 1 to 1000 rows, K
+    // 256 to 4096 and 256 to 4096 columns (E4M3 and FP4 W, fp32 and bf16 x), each
+    // run both ways, these lines are 0.8% from the better one on average and more
+    // than a fifth on 27, all of them a K of 2100 or 3000 with several workgroups a
+    // CU, or 1536 with at most 16 rows; without quads 5.9%, with them wherever they
+    // can run 6.4%.
     if constexpr (dtype_bits(WT) <= 16) {
       const int64_t tiles32 = ((M + 31) / 32) * ((N + 31) / 32);
       if (M >= 4 && M <= 16 && K >= 2048)
