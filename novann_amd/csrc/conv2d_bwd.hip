@@ -183,14 +183,17 @@ __global__ __launch_bounds__(256) void zero_kernel(float* __restrict__ p, int64_
 // outside grad is skipped, not multiplied by zero.  by_tap: only the phases
 // that a tap reaches are run, on a zeroed grad_input.
 //
-// Bound by the LDS pipe (four broadcast reads to 16 products; two pixels a
-// lane need a select a product for the taps only one of them has: 271 us
-// against 181).  Where 256 pixels a workgroup would leave CUs idle (SPLIT) the
-// waves take a quarter of each stage's output channels of the same 64 pixels
-// and their sums are added in wave order.  Measured (E4M3, 64 <- 128 channels,
+// Bound by the LDS and VALU pipes together (four broadcast reads to 16 products:
+// LDS 59% busy, 0.78 VALU instructions a cycle; two pixels a lane need a select a
+// product for the taps only one of them has: 271 us against 181) and by memory:
+// a layer reads the grad again and a phase writes every second pixel of a line,
+// 472 MB read and 118 written for 25.7 and 51.4 at the size below.  Where 256
+// pixels a workgroup would leave CUs idle (SPLIT) the waves take a quarter of
+// each stage's output channels of the same 64 pixels and their sums are added in
+// wave order.  Measured (E4M3, 64 <- 128 channels,
 // 3 x 3 / 2, 256 maps of 28 x 28): 181 us, 4414 with one lane an element that
-// decoded every weight for itself; 256 <- 256 channels, 8 maps of 7 x 7: 54.7
-// us (301; 147 without SPLIT).
+// decoded every weight for itself (200 in a kernel trace on another card); 256 <-
+// 256 channels, 8 maps of 7 x 7: 54.7 us (301; 147 without SPLIT).
 constexpr int DI_CO = 128;  // output channels a stage
 template <int WT, int CT, bool SPLIT>
 __global__ __launch_bounds__(256) void dinput_phase_kernel(const float* __restrict__ grad,

@@ -865,7 +865,8 @@ __device__ __forceinline__ void pool_stage(const uint8_t* __restrict__ x, int64_
 // as max_pool2d_bwd_kernel's.  K, S: square windows of K and stride S fixed at
 // compile time (0: the geometry's), which takes the loops' bounds and the
 // divisions by the stride out (57.0 -> 49.8 us).  VALU-bound on the index
-// arithmetic; measured (256 x 64 planes of 28 x 28, fp32): 3 x 3 / 2 with
+// arithmetic (1.16 VALU instructions a busy CU cycle, about all that four SIMDs
+// take; the LDS is busy 23%); measured (256 x 64 planes of 28 x 28, fp32): 3 x 3 / 2 with
 // padding 49.8 us, 491 on max_pool2d_bwd_kernel's one-lane-an-element walk;
 // 3 x 3 / 1 88.1 us (1024).
 template <int XT, int K, int S>
